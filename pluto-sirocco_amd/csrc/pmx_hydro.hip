@@ -152,12 +152,80 @@ struct pmx_hydro {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pending;
   double timed_ms;
   int timed_launches;
-  int cz;
 };
 
 namespace {
 
-int z_schedule(int nz, int* zc0);
+// The z chunks of a 3-D grid of `tiles` x-y tiles.
+struct ZPlan {
+  int n;                          // chunks of zc0, or 0: uniform chunks of cz planes
+  int zc0[PMX_MAX_ZCHUNKS + 1];
+  int cz;
+};
+
+// z chunks of decreasing length: `size` planes while more than 2 size
+// remain, then half of that, ..., then pieces of `least` planes (nz = 256,
+// 64 and 8: 64, 64, 32, 32, 16, 16, 8, 8, 8, 8), long ones dispatched
+// first.  Returns the number of chunks, or 0 when they do not fit zc0.
+int z_decreasing(int nz, int size, int least, int* zc0) {
+  int n = 0, z = 0, rem = nz;
+  auto push = [&](int len) { zc0[n++] = z; z += len; rem -= len; };
+  for (; size >= least; size /= 2)
+    while (rem > 2 * size && n < PMX_MAX_ZCHUNKS) push(size);
+  while (rem > 0 && n < PMX_MAX_ZCHUNKS) push(rem < least ? rem : least);
+  zc0[n] = nz;
+  return rem == 0 ? n : 0;
+}
+
+// How the z planes are cut among workgroups.  256 CUs hold two workgroups
+// each; a chunk of L planes costs a workgroup L + 1.45 plane times (the
+// ghost planes, two states and a face of its start), a plane taking 8.3 us
+// next to a second workgroup of the CU and 5.5 us alone (PPM + HLLC).  Two
+// plans are priced that way and the cheaper one is taken:
+//  * one round: equal chunks, as many as let every workgroup be resident
+//    at once (or one per CU).  It suits grids of few tiles, whose launch
+//    would otherwise last as long as its longest chunk: per stage 64^3
+//    (20 tiles) takes 37 us in 3-plane chunks against 101 us in chunks of
+//    16 .. 8, 101 x 66 x 93 (35 tiles) 73 us in 7-plane chunks against 193;
+//  * chunks of decreasing length, the longest at most 7/16 of the planes a
+//    slot gets: long chunks cost less in re-read ghost planes, the short
+//    ones dispatched last let every CU finish together.  Sedov 256^3 (64 ..
+//    8): 1.265 ms per stage, equal 16-plane chunks 1.311, 32-plane ones
+//    1.354.
+// PMX_CZ sets uniform chunks of its own.
+ZPlan z_plan(int tiles, int nz) {
+  ZPlan p;
+  p.n = 0;
+  p.cz = nz < 64 ? 8 : 16;
+  if (const char* e = getenv("PMX_CZ")) {
+    p.cz = atoi(e) > 0 ? atoi(e) : p.cz;
+    return p;
+  }
+  const int cus = 256, slots = 2 * cus;
+  const double start = 1.45, alone = 0.66;
+  double best = 1e300;
+  for (int fit : {slots, cus}) {
+    const int n = std::min(fit / tiles, nz);
+    if (n < 1) continue;
+    const int len = (nz + n - 1) / n;
+    const double t = (len + start) * (tiles * ((nz + len - 1) / len) <= cus ? alone : 1.0);
+    if (t < best) { best = t; p.cz = len; }
+  }
+  const double share = (double)tiles * nz / slots;   // planes per slot
+  int size = 64;
+  while (size > 2 && size > share * 0.4375) size /= 2;
+  const int least = std::min(8, std::max(2, size / 2));
+  p.n = z_decreasing(nz, size, least, p.zc0);
+  if (p.n == 0) {                  // a column too long for zc0
+    if (best > 1e299) p.cz = size;
+    return p;
+  }
+  // later rounds overlap the starts of their chunks with other workgroups'
+  // planes: 0.6 planes per chunk, and 0.87 of the price of one round
+  const double t = 0.87 * (tiles * (nz + 0.6 * p.n) / slots + 0.5 * (least + start));
+  if (best <= t) p.n = 0;
+  return p;
+}
 
 // The boundary kind of a domain: one rule on every side of the active
 // directions is compiled in (BCK_OUTFLOW, BCK_PERIODIC), else BCK_ANY.
@@ -227,12 +295,19 @@ int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int m
   a.dtdx[0] = h->dtdx; a.dtdx[1] = h->dtdx + h->nx; a.dtdx[2] = h->dtdx + h->nx + h->ny;
   a.inv_dl[0] = h->inv_dl; a.inv_dl[1] = h->inv_dl + h->nx; a.inv_dl[2] = h->inv_dl + h->nx + h->ny;
   a.w0 = w0; a.wc = wc;
-  a.cz = h->cz;
   a.tiles_x = (h->nx + TILE_X - 1) / TILE_X;
   const int ty = h->d.dims == 3 ? tile_y<3>() : tile_y<2>();
   a.tiles_y = (h->ny + ty - 1) / ty;
-  a.nzc = h->d.dims == 3 ? z_schedule(h->nz, a.zc0) : 0;
-  a.tiles_z = (h->d.dims == 3) ? (a.nzc ? a.nzc : (h->nz + h->cz - 1) / h->cz) : 1;
+  a.nzc = 0;
+  a.cz = 1;
+  a.tiles_z = 1;
+  if (h->d.dims == 3) {
+    const ZPlan p = z_plan(a.tiles_x * a.tiles_y, h->nz);
+    a.nzc = p.n;
+    if (p.n) memcpy(a.zc0, p.zc0, sizeof(int) * (p.n + 1));
+    a.cz = p.cz;
+    a.tiles_z = p.n ? p.n : (h->nz + p.cz - 1) / p.cz;
+  }
   a.write_u = write_u;
   a.cdt_bits = h->s->cdt_red;
   a.err = &h->s->err;
@@ -358,37 +433,6 @@ int check_desc(const pmx_hydro_desc* desc) {
   return 0;
 }
 
-// z planes per workgroup: long enough to amortise the column prologue,
-// short enough to give several workgroups per CU.  PMX_CZ overrides.
-int z_chunk(int nz) {
-  int cz = nz < 64 ? 8 : 16;
-  if (const char* e = getenv("PMX_CZ")) cz = atoi(e) > 0 ? atoi(e) : cz;
-  return cz;
-}
-
-// z chunks of decreasing length for a 3-D grid: 64 planes while more than
-// 128 remain, then 32 while more than 64, 16 while more than 32, 8 while
-// more than 16, then 8-plane pieces (nz = 256: 64, 64, 32, 32, 16, 16, 8,
-// 8, 8, 8).  Each chunk re-reads 3 + 3 ghost planes and redoes two z
-// states and a z face per column, so long chunks cost less; but a launch
-// of equal chunks leaves its last round of workgroups partly empty (Sedov
-// 256^3 in 16-plane chunks: 4,864 workgroups, 512 resident at a time, 9.5
-// rounds), whereas short chunks dispatched last let every CU finish
-// together: 1.265 vs 1.311 ms per stage (32-plane chunks first: 1.273;
-// equal 32-plane chunks: 1.354).  Writes zc0[0..n] (zc0[n] = nz) and
-// returns the number n of chunks, or 0 for the uniform chunks of z_chunk
-// (PMX_CZ set, or more chunks than fit).
-int z_schedule(int nz, int* zc0) {
-  if (getenv("PMX_CZ")) return 0;
-  int n = 0, z = 0, rem = nz;
-  auto push = [&](int len) { zc0[n++] = z; z += len; rem -= len; };
-  for (int size = 64; size >= 8; size /= 2)
-    while (rem > 2 * size && n < PMX_MAX_ZCHUNKS) push(size);
-  while (rem > 0 && n < PMX_MAX_ZCHUNKS) push(rem < 8 ? rem : 8);
-  zc0[n] = nz;
-  return rem == 0 ? n : 0;
-}
-
 // dx per cell of every direction ([nx | ny | nz]) and its reciprocal
 // (Src/set_geometry.c:305).
 void host_tables(const pmx_hydro_desc* desc, int nx, int ny, int nz, std::vector<double>& dx,
@@ -416,7 +460,6 @@ int pmx_hydro_create(const pmx_hydro_desc* desc, pmx_hydro** out) {
   h->d = *desc;
   h->nx = desc->nx1; h->ny = desc->nx2; h->nz = nz;
   h->ncell = (long long)h->nx * h->ny * h->nz;
-  h->cz = z_chunk(h->nz);
   size_t vbytes = sizeof(double) * NV * h->ncell;
   int ntot = h->nx + h->ny + h->nz;
 #define CK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { \
@@ -710,7 +753,6 @@ int pmx_hydro_advance_step_noalloc(const pmx_hydro_desc* desc, double* V, double
   h.d = *desc;
   h.nx = nx; h.ny = ny; h.nz = nz;
   h.ncell = ncell;
-  h.cz = z_chunk(nz);
   h.V[0] = V;
   h.V[1] = base;
   h.V[2] = base + (size_t)NV * ncell;
