@@ -554,8 +554,10 @@ int pmx_copy_probe_runtime(long long nbytes, int reps, double *ms_per_copy);
  * line_connect.c:753 and :899-900) are evaluated from a reciprocal with
  * FMA corrections where the run's inputs keep the operands in range; this
  * runs that evaluation and the plain division of each of the n values x
- * (0, or |x| and |x / c| within 2^-900..2^900) by c > 0 on the device and
- * reports how many of the quotients differ in any bit (0 expected). */
+ * (0, or |x| and |x / c| within 2^-900..2^900) by c > 0 on the device, and
+ * the line force's other quotient forms and square root of the same values,
+ * and reports how many of the x have a result that differs in any bit (0
+ * expected). */
 int pmx_check_div_rc(const double *x, long long n, double c, long long *mismatches);
 
 /* Arithmetic check (no counterpart in the reference): the line force's

@@ -24,6 +24,58 @@ __device__ __forceinline__ double minmod(double a, double b) {                  
   return a * b > 0.0 ? (fabs(a) < fabs(b) ? a : b) : 0.0;
 }
 
+// ---------------------------------------------------------------------
+// Division and square root for operands of moderate exponent: the Newton /
+// Goldschmidt steps alone, without the operand scaling and the special
+// cases (0, inf, NaN, subnormal) of the general operations, 7 instructions
+// against 11 and 8 against 17.  recip(d) serves every quotient with that
+// divisor (3 instructions each).  The quotient is the IEEE one while divisor,
+// dividend and quotient lie in about 2^-900 .. 2^900 (dividend 0 included,
+// up to the sign of the zero), and so is the root while its argument does:
+// the hardware's first estimate has some 26 bits, the cubic step (the
+// coupled quadratic one of the root) brings it to the last bit, the
+// residual is exact in the FMA, and the corrected value is rounded once.
+// pmx_check_div_rc compares them with the general operations.
+// ---------------------------------------------------------------------
+__host__ __device__ __forceinline__ double recip(double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+#else
+  return 1.0 / d;
+#endif
+}
+// n / d, given y = recip(d)
+__host__ __device__ __forceinline__ double quot(double n, double d, double y) {
+  const double q = n * y;
+  return fma(fma(-d, q, n), y, q);
+}
+// sqrt(x); y becomes 1 / sqrt(x) to a few ulps
+__host__ __device__ __forceinline__ double sqrt_mod(double x, double& y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r = __builtin_amdgcn_rsq(x);
+  double g = x * r, h = r * 0.5;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, x), h, g);
+  y = h + h;
+  return g;
+#else
+  y = 1.0 / sqrt(x);
+  return sqrt(x);
+#endif
+}
+
+// A constant held in scalar registers: an FMA then takes it from there,
+// where the compiler would otherwise copy it to vector registers (two
+// moves) at every use in a loop.
+__device__ __forceinline__ double scalar_const(double c) {
+  asm("" : "+s"(c));
+  return c;
+}
+
 // Src/HD/mappers.c:44-57 (EOS IDEAL)
 __device__ __forceinline__ void prim_to_cons(const double* v, double* u, double gmm1) {
   double rho = v[RHO];

@@ -484,6 +484,162 @@ __device__ __forceinline__ void lforce_cell(const StageArgs& a, int i, int j) {
   a.glf[a.sv + cell] = g2t;
 }
 
+// ---------------------------------------------------------------------
+// The same line force, bit for bit (see force_mult_fast), for grids whose
+// inputs keep the operands' exponents moderate (k.lf_fast, decided at
+// create: the reference's power with |alpha| <= 2 and krad >= 0, fluxes,
+// radii and offset lengths within the ranges stated there).  The bin loop is
+// bound by VALU issue: two wavefronts per SIMD fill it, one by itself waits
+// twice as long for its own results.  This form is the one with few
+// instructions, 267 per bin against 445 of lforce_cell: quotients and roots
+// without scaling, reciprocals shared, the root's serving the division by
+// ds, one straight-line block for both powers, coefficients in scalar
+// registers.  512 x 256: 89 -> 62 us per launch (24.8 M instead of 32.8 M
+// wave instructions at the first of its steps, 21.5 M now).
+// dvds is range-checked over the loop; a zone with one outside (or with such
+// a num) takes its bins again in the general form.
+// ---------------------------------------------------------------------
+struct LfCell {
+  VGrad vg;
+  double num1, num2;
+};
+
+// x / c for a c that many quotients share: r + l = 1 / c to twice the
+// precision, so that the first quotient is within an ulp and one correction
+// rounds it (Markstein).  The sign of a zero is that of the dividend's only
+// when it is positive, which the sums these quotients go into do not see.
+struct Recip2 {
+  double c, r, l;
+};
+
+__device__ __forceinline__ Recip2 recip2(double c, double r) {   // r = 1 / c, rounded
+  return {c, r, fma(-c, r, 1.0) * r};
+}
+
+__device__ __forceinline__ double div2(double x, const Recip2& k) {
+  const double q = fma(x, k.r, x * k.l);
+  return fma(fma(-q, k.c, x), k.r, q);
+}
+
+constexpr double LF_HI = 0x1p400;    // range of dvds: 0, or 2^-400 .. 2^400
+constexpr int LF_NMAX = 400;
+constexpr double LF_NUM_LO = 0x1p-100, LF_NUM_HI = 0x1p100;
+
+// The zone's part: both calls' num and the VGradCalc corners.
+template <int FEAT>
+__device__ __forceinline__ void lforce_zone(const StageArgs& a, int i, int j, LfCell& z) {
+  const Const& k = a.k;
+  double vc[NVW], w1[NVW], e1[NVW], c[6], vpi[NVW], vmi[NVW];
+  ld6(a, a.Vin, j, i, vc);
+  ld6(a, j, i - 1, w1);
+  ld6(a, j, i + 1, e1);
+  ldc(a.T.pr, a.nr, i + NG, c);
+  plm_zone<0, FEAT & FEAT_CHAR>(a, j, i, w1, vc, e1, c, vpi, vmi);
+  const double r1 = 0.5 * (vpi[RHO] + vmi[RHO]), p1 = 0.5 * (vpi[PRS] + vmi[PRS]);
+  const double rho1 = r1 * k.UD, rho2 = vc[RHO] * k.UD;
+  const double T1 = p1 / r1 * k.KELVIN * k.mu;
+  const double T2 = vc[PRS] / vc[RHO] * k.KELVIN * k.mu;
+  const double vth1 = sqrt((2.0 * C_kB * T1) / C_mp);
+  const double vth2 = sqrt((2.0 * C_kB * T2) / C_mp);
+  z.num1 = k.sigma_e * rho1 * vth1;
+  z.num2 = k.sigma_e * rho2 * vth2;
+  vgrad_cell(a, j, i, z.vg);
+}
+
+// The zone's bins ang0, ang0 + step, ...: f(ang, g_r term, g_theta term);
+// restart() before f is called for the same bins again.
+template <class F, class R>
+__device__ __forceinline__ void lforce_bins(const StageArgs& a, const LfCell& z, unsigned cell,
+                                            int ang0, int step, F f, R restart) {
+  if (ang0 >= a.na) return;
+  const Const& k = a.k;
+  const VGrad& g = z.vg;
+  const long long sa = a.sv * a.na;
+  const unsigned off = cell * 8u;          // byte offset of the zone in a table plane
+  // (the offset opaque, so that the load takes the plane from scalar
+  // registers instead of a 64-bit address formed per entry)
+  auto entry = [&](int t, int ang) {
+    const char* plane = reinterpret_cast<const char*>(a.T.lf + t * sa + ang * a.sv);
+    unsigned o = off;
+    asm("" : "+v"(o));
+    return *reinterpret_cast<const double*>(plane + o);
+  };
+  bool bad = !(z.num1 >= LF_NUM_LO && z.num1 <= LF_NUM_HI && z.num2 >= LF_NUM_LO &&
+               z.num2 <= LF_NUM_HI);
+  {
+    const PowSeries C = pow_series();
+    PowNum P[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      int n;
+      P[q].num = q ? z.num2 : z.num1;
+      P[q].rn = LOG2E_HI / P[q].num;
+      P[q].L = log2_dd_fast(P[q].num, C, n);
+    }
+    const Recip2 dx0 = recip2(g.dx0, g.rdx0), rc = recip2(C_c, 1.0 / C_c),
+                 ua = recip2(k.UA, 1.0 / k.UA);
+    double dmax_ = 0.0;                  // largest dvds, and the smallest's scaling
+    int nmax = 0;
+    auto bin = [&](int ang) {
+      const double st = a.T.sta[ang], ct = a.T.cta[ang];
+      const double g2 = entry(LF_F2, ang), so = entry(LF_SIN, ang), co = entry(LF_COS, ang);
+      const double fr = entry(LF_FR, ang), ft = entry(LF_FT, ang);
+      const double ddx1 = g.maxds * st, ddx2 = g.maxds * ct;
+      double rds, rr;
+      const double ds = sqrt_mod(ddx1 * ddx1 + ddx2 * ddx2, rds);
+      const double roff = sqrt_mod((g.x + ddx1) * (g.x + ddx1) + (g.z + ddx2) * (g.z + ddx2), rr);
+      const double g1 = div2(roff - g.x11_0, dx0);
+      const double h1 = 1.0 - g1, h2 = 1.0 - g2;
+      const double b0 = h2 * (h1 * g.v11_0 + g1 * g.v21_0) + g2 * (h1 * g.v12_0 + g1 * g.v22_0);
+      const double b1 = h2 * (h1 * g.v11_1 + g1 * g.v21_1) + g2 * (h1 * g.v12_1 + g1 * g.v22_1);
+      const double b0u = b0 * k.UV, b1u = b1 * k.UV;
+      const double vx2 = b0u * so + b1u * co;
+      const double vz2 = b0u * co - b1u * so;
+      const double u1 = st * g.vx1 + ct * g.vz1;
+      const double u2 = st * vx2 + ct * vz2;
+      rds = fma(rds, fma(-ds, rds, 1.0), rds);
+      // a bin without flux (g2 = -999) has a dvds too, and an M that its
+      // zero fluxes annul
+      const double dvds = fabs(quot(u2 - u1, ds, rds));
+      int n;
+      const DD D = log2_dd_fast(dvds, C, n);
+      dmax_ = fmax(dmax_, dvds);
+      nmax = max(nmax, n);
+      const double y = recip(dvds);
+      const double f1 = 1.0 + force_mult_fast(k, P[0], dvds, y, D, C);
+      const double f2 = 1.0 + force_mult_fast(k, P[1], dvds, y, D, C);
+      // ((fm sigma_e f) / c) / UA, each quotient bit-identical
+      f(ang, div2(div2(f1 * k.sigma_e * fr, rc), ua),
+        div2(div2(f2 * k.sigma_e * ft, rc), ua));
+    };
+#pragma unroll 1
+    for (int ang = ang0; ang < a.na; ang += step) bin(ang);
+    // (dvds = 0 has n = 1, inf and NaN too: inf shows in dmax_, and a NaN
+    // gets M = 0 as in the reference)
+    bad = bad | !(dmax_ <= LF_HI) | (nmax > LF_NMAX);
+  }
+  if (!bad) return;
+  restart();      // the general form
+  const double n1 = z.num1, n2 = z.num2;
+#pragma unroll 1
+  for (int ang = ang0; ang < a.na; ang += step) {
+    const double dvds = vgrad_dvds(a, g, entry(LF_F2, ang), entry(LF_SIN, ang),
+                                   entry(LF_COS, ang), ang);
+    double t1 = 0.0, t2 = 0.0;
+#pragma unroll 1
+    for (int call = 0; call < 2; call++) {
+      double M = 0.0;
+      if (dvds > 0.0) {
+        M = force_power_shared(k, pow_num(call ? n2 : n1), dvds, log2_dd(dvds));
+        if (M > 4400.) M = 4400.;
+      }
+      t1 = t2;
+      t2 = (1.0 + M) * k.sigma_e * entry(call ? LF_FT : LF_FR, ang) / C_c / k.UA;
+    }
+    f(ang, t1, t2);
+  }
+}
+
 template <int STAGE, int FEAT>
 __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, double& cdt,
                                            int& flags) {
@@ -815,6 +971,64 @@ __global__ __launch_bounds__(BX* BY) void wind_lforce_kernel(StageArgs a) {
   const int i = blockIdx.x * BX + threadIdx.x;
   const int j = blockIdx.y * BY + threadIdx.y;
   if (i < a.nr && j < a.nt) lforce_cell<FEAT>(a, i, j);
+}
+
+template <int FEAT>
+__device__ __forceinline__ void lforce_zone_bins(const StageArgs& a, unsigned cell) {
+  const int j = cell / (unsigned)a.nr, i = cell - j * a.nr;
+  LfCell z;
+  lforce_zone<FEAT>(a, i, j, z);
+  double g1r = 0.0, g2t = 0.0;
+  lforce_bins(
+      a, z, cell, 0, 1,
+      [&](int, double t1, double t2) {
+        g1r += t1;
+        g2t += t2;
+      },
+      [&] { g1r = g2t = 0.0; });
+  a.glf[cell] = g1r;
+  a.glf[a.sv + cell] = g2t;
+}
+
+// The line force through lforce_bins.  The threads run over the flattened
+// zone index, so that only the last wavefront has idle lanes and a
+// wavefront's table loads are contiguous whatever nr is (200 x 100: 32 us
+// against 52 with rows of their own, 301 x 143: 50 against 59).
+template <int FEAT>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void wind_lforce_fast_kernel(StageArgs a) {
+  if (a.loop && a.s->halt) return;     // uniform over the launch
+  const unsigned cell = blockIdx.x * 128 + threadIdx.x;
+  if (cell < a.sv) lforce_zone_bins<FEAT>(a, cell);
+}
+
+// The same with a zone's bins shared by S wavefronts: the terms meet in LDS
+// and are added in bin order.
+template <int FEAT, int S>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3)))
+void wind_lforce_split_kernel(StageArgs a) {
+  extern __shared__ double terms[];    // [na][2][64]
+  if (a.loop && a.s->halt) return;     // uniform over the launch
+  const unsigned cell = blockIdx.x * 64 + threadIdx.x;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  if (cell < a.sv) {
+    const int j = cell / (unsigned)a.nr, i = cell - j * a.nr;
+    LfCell z;
+    lforce_zone<FEAT>(a, i, j, z);
+    lforce_bins(
+        a, z, cell, s, S,
+        [&](int ang, double t1, double t2) {
+          terms[(2 * ang) * 64 + threadIdx.x] = t1;
+          terms[(2 * ang + 1) * 64 + threadIdx.x] = t2;
+        },
+        [] {});
+  }
+  __syncthreads();
+  if (cell < a.sv && s < 2) {
+    double sum = 0.0;
+    for (int ang = 0; ang < a.na; ang++) sum += terms[(2 * ang + s) * 64 + threadIdx.x];
+    a.glf[s * a.sv + cell] = sum;
+  }
 }
 
 template <int MODE>
@@ -1174,8 +1388,30 @@ void launch_feat(pmx_wind* w, dim3 grid, dim3 block, const StageArgs& a) {
     hipLaunchKernelGGL((wind_stage_kernel<STAGE, FEAT>), grid, block, 0, w->stream, a);
 }
 
+// Four wavefronts share the bins of 64 zones while the zones alone make
+// fewer than one and a half wavefronts per SIMD (8 k cells: 15 against 30 us,
+// 43 k: 29 against 50, 74 k: 45 against 52, 98 k: 54 both ways, 131 k: 75
+// against 62; two or eight wavefronts measured slower from 20 k cells on).
+constexpr long long LF_SPLIT_CELLS = 3 * 64 * 1024 / 2;
+
+template <int FEAT>
+void launch_lforce_fast(pmx_wind* w, const StageArgs& a) {
+  if (w->sv < LF_SPLIT_CELLS) {
+    const size_t lds = sizeof(double) * 2 * 64 * w->na;     // 64 KiB at most
+    hipLaunchKernelGGL((wind_lforce_split_kernel<FEAT, 4>), dim3((unsigned)((w->sv + 63) / 64)),
+                       dim3(64, 4), lds, w->stream, a);
+  } else {
+    hipLaunchKernelGGL((wind_lforce_fast_kernel<FEAT>), dim3((unsigned)((w->sv + 127) / 128)),
+                       dim3(128), 0, w->stream, a);
+  }
+}
+
 template <int STAGE>
 void launch_stage(pmx_wind* w, dim3 grid, dim3 block, const StageArgs& a) {
+  if (w->k.lf_fast) {
+    if (w->k.char_lim) launch_lforce_fast<FEAT_CHAR>(w, a);
+    else launch_lforce_fast<0>(w, a);
+  } else
   switch (features(w) & (FEAT_CHAR | FEAT_TAB)) {
     case 0: hipLaunchKernelGGL((wind_lforce_kernel<0>), grid, block, 0, w->stream, a); break;
     case FEAT_CHAR:
@@ -1305,21 +1541,27 @@ Const make_const(const pmx_wind_desc* d) {
   k.roe = d->solver == PMX_SOLVER_ROE;
   k.first_dt = d->first_dt;
   k.fm_points = (d->krad == 999 && d->alpharad == 999) ? d->fm_points : 0;
-  k.fast_div = 0;   // set with the line-force tables
+  k.fast_div = k.lf_fast = 0;   // set with the line-force tables
   k.fm_fast = d->force_power == PMX_FORCE_POWER_FACTORED;
   k.midplane = 0;   // set with the geometry
   return k;
 }
 
-// div_rc against the division on the device: the count of x whose two
-// quotients differ in any bit.
+// div_rc, quot, div2 and sqrt_mod against the division and the root on the
+// device: the count of x with a result that differs in any bit (zero
+// quotients of the latter two in value only).
 __global__ void div_check_kernel(const double* __restrict__ x, long long n, double c, double rc,
                                  unsigned long long* bad) {
   unsigned long long mine = 0;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     const double q = div_rc(x[i], c, rc), r = x[i] / c;
-    if (__double_as_longlong(q) != __double_as_longlong(r)) mine++;
+    bool same = __double_as_longlong(q) == __double_as_longlong(r);
+    same = same && quot(x[i], c, recip(c)) == r && div2(x[i], recip2(c, rc)) == r;
+    const double ax = fabs(x[i]);
+    double y;
+    if (ax > 0.0) same = same && sqrt_mod(ax, y) == sqrt(ax);
+    if (!same) mine++;
   }
   if (mine) atomicAdd(bad, mine);
 }
@@ -1502,6 +1744,7 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
     const double af = fabs(f);
     return af == 0.0 || (af >= 0x1p-600 && af <= 0x1p600);
   };
+  bool lf_geom = true;
   bool fast_div = k.UA >= 0x1p-100 && k.UA <= 0x1p100;
   for (int I = 0; I < nr + 2 * NG; I++) {
     const double r = x1[I] * UL;
@@ -1519,6 +1762,8 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
         maxds /= 2.0;
         double fr = d->flux_r[q], ft = d->flux_t[q], fp = d->flux_p[q];
         if (!div_rc_flux_ok(fr) || !div_rc_flux_ok(ft)) fast_div = false;
+        // the roots of lforce_cell_fast: the offset length and radius
+        if (!(maxds >= 0x1p-300 && maxds <= 0x1p300)) lf_geom = false;
         double mod_flux = sqrt(pow(fr, 2) + pow(ft, 2) + pow(fp, 2));
         lf[LF_FR * sa + q] = fr;
         lf[LF_FT * sa + q] = ft;
@@ -1529,6 +1774,8 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
         double x = x1[I] * sin(x2[J]) * UL, z = x1[I] * cos(x2[J]) * UL;
         double ta = (a + 0.5) * (2.0 * C_PI) / 36.0;
         double ddx1 = maxds * sin(ta), ddx2 = maxds * cos(ta);
+        const double roff2 = (x + ddx1) * (x + ddx1) + (z + ddx2) * (z + ddx2);
+        if (!(roff2 >= 0x1p-600 && roff2 <= 0x1p600)) lf_geom = false;
         // ds and the radial weight (roff - x11_0) / (x22_0 - x11_0) are
         // recomputed per bin by the stage (vgrad_dvds), bit for bit
         double toff = atan((x + ddx1) / (z + ddx2));
@@ -1537,6 +1784,8 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
         lf[LF_COS * sa + q] = cos(toff);
       }
   w->k.fast_div = fast_div ? 1 : 0;
+  w->k.lf_fast = fast_div && lf_geom && !w->k.fm_fast && w->k.fm_points == 0 &&
+                 fabs(k.alpharad) <= 2.0 && k.krad >= 0.0 && k.krad <= 0x1p100;
 
   // pack the geometry tables into one buffer
   std::vector<std::pair<const double**, const std::vector<double>*>> parts = {
@@ -2002,6 +2251,20 @@ __global__ __launch_bounds__(TBX* TBY) void wind_batch_lforce_kernel(
   }
 }
 
+// The same through lforce_bins, over the grids' flattened zones (off: each
+// grid's first zone, a multiple of 128).
+template <int FEAT>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void wind_batch_lforce_fast_kernel(const StageArgs* __restrict__ args,
+                                   const long long* __restrict__ off, int G) {
+  const long long q = (long long)blockIdx.x * 128;
+  const int g = __builtin_amdgcn_readfirstlane(find_grid(off, G, q));
+  const StageArgs& a = args[g];
+  if (a.s->halt) return;               // a halted grid (uniform over the workgroup)
+  const unsigned cell = (unsigned)(q - off[g]) + threadIdx.x;
+  if (cell < a.sv) lforce_zone_bins<FEAT>(a, cell);
+}
+
 // Per grid: fold the stage-1 C_dt into invDt (update_stage.c:389-394),
 // t += dt, and NextTimeStep + reset when `next` (see wind_end_kernel).
 __global__ __launch_bounds__(64) void wind_batch_end_kernel(const StageArgs* args, int G, int next,
@@ -2070,6 +2333,7 @@ struct pmx_wind_batch {
   long long cells;        // interior cells of all grids
   int feat_any;           // OR of the grids' features (characteristic limiting, the entropy
                           // switch, the tabulated force multiplier, Roe)
+  int lf_fast;            // every grid's line force through lforce_bins
   int shape;              // index into the tile-shape table
   int blocks;             // persistent workgroups per stage launch
   hipStream_t stream;
@@ -2096,9 +2360,19 @@ template <int STAGE>
 void launch_batch_stage(pmx_wind_batch* b) {
   const StageArgs* args = STAGE == 1 ? b->args1 : b->args2;
   const dim3 grid(b->blocks);
+  if (b->lf_fast) {
+    const dim3 lg((unsigned)(b->total_cells / 128));
+    if (b->feat_any & FEAT_CHAR)
+      hipLaunchKernelGGL((wind_batch_lforce_fast_kernel<FEAT_CHAR>), lg, dim3(128), 0, b->stream,
+                         args, b->cell_off, b->G);
+    else
+      hipLaunchKernelGGL((wind_batch_lforce_fast_kernel<0>), lg, dim3(128), 0, b->stream, args,
+                         b->cell_off, b->G);
+  }
 #define PMX_SHAPE(q, X, Y)                                                                   \
   case q:                                                                                    \
-    if (b->feat_any)                                                                         \
+    if (b->lf_fast) ;                                                                        \
+    else if (b->feat_any)                                                                    \
       hipLaunchKernelGGL((wind_batch_lforce_kernel<FEAT_CHAR | FEAT_TAB, X, Y>), grid,       \
                          dim3(X, Y), 0, b->stream, args, b->tile_off, b->G, b->total_tiles); \
     else                                                                                     \
@@ -2252,8 +2526,10 @@ int pmx_wind_batch_create(const pmx_wind_desc* descs, int ngrids, pmx_wind_batch
   std::vector<double> cfl(G), cmv(G);
   std::vector<long long> coff(G + 1, 0);
   b->cells = 0;
+  b->lf_fast = 1;
   for (int g = 0; g < G; g++) {
     pmx_wind* w = b->grids[g];
+    if (!w->k.lf_fast) b->lf_fast = 0;
     a1[g] = stage_args(w, w->V[0], w->V[1], true);
     a2[g] = stage_args(w, w->V[1], w->V[0], true);
     ca[g] = cool_args(w);

@@ -55,6 +55,7 @@ struct Const {
   int hll;                                 // [Solver] hll instead of hllc
   int roe;                                 // [Solver] roe
   int fast_div;                            // line-force quotients through div_rc
+  int lf_fast;                             // the line force through lforce_cell_fast
   int fm_fast;                             // factored force-multiplier power (see force_mult_pair)
   double first_dt;                         // runtime->first_dt (dt-too-small stop)
   int fm_points;                           // > 0: tabulated force multiplier (krad = alpharad = 999)
@@ -484,6 +485,94 @@ PMX_HD void force_mult_shared(const Const& k, const PowNum& a1, const PowNum& a2
   }
   f1 = 1.0 + M1;
   f2 = 1.0 + M2;
+}
+
+// ---------------------------------------------------------------------
+// force_mult_shared for operands of moderate exponent with fewer
+// instructions (see lforce_bins): the logarithm's two quotients share a
+// reciprocal, and so do both calls' t; Fast2Sum where the larger operand is
+// known (in t's logarithm: unless t is within 2^-48 of 1, where what it
+// drops is below 2^-100); FMAs in the low-order terms; no special cases;
+// the series' coefficients in scalar registers.  What changes against
+// force_mult_shared lies below 2^-100 of the result before its last
+// rounding, so the two agree in every bit but for one argument in 2^45 or so.
+// ---------------------------------------------------------------------
+PMX_HD DD dd_fast_sum(double a, double b) {   // a + b exactly, |a| >= |b| or a == 0
+  const double s = a + b;
+  return {s, b - (s - a)};
+}
+
+// The atanh series 1/3 .. 1/23, the Taylor series 1/2! .. 1/14!, 2 log2 e,
+// ln 2 and the root of 2
+struct PowSeries {
+  double la[11], ex[13], l2h, l2l, n2h, n2l, root2;
+};
+
+__device__ __forceinline__ PowSeries pow_series() {
+  PowSeries c;
+#pragma unroll
+  for (int q = 0; q < 11; q++) c.la[q] = scalar_const(1.0 / (23.0 - 2.0 * q));
+  double f = 2.0;
+#pragma unroll
+  for (int q = 0; q < 13; q++) {   // ex[12] = 1/2! (an inline constant), ex[0] = 1/14!
+    c.ex[12 - q] = q ? scalar_const(1.0 / f) : 0.5;
+    f *= (double)(q + 3);
+  }
+  c.l2h = scalar_const(2.0 * LOG2E_HI);
+  c.l2l = scalar_const(2.0 * LOG2E_LO);
+  c.n2h = scalar_const(LN2_HI);
+  c.n2l = scalar_const(LN2_LO);
+  c.root2 = scalar_const(1.4142135623730951);
+  return c;
+}
+
+// log2_dd for a normal x, x 2^n in [sqrt(1/2), sqrt(2))
+__device__ __forceinline__ DD log2_dd_fast(double x, const PowSeries& c, int& n) {
+  n = 1 - __builtin_amdgcn_frexp_exp(x * c.root2);
+  const double m = ldexp(x, n);
+  const double a = m - 1.0;
+  const DD b = dd_fast_sum(1.0, m);        // exponent of m at most that of 1
+  const double y = recip(b.hi);
+  const double sh = quot(a, b.hi, y);
+  const double sl = (fma(-sh, b.hi, a) - sh * b.lo) * y;
+  const double z = sh * sh;
+  double p = c.la[0];
+#pragma unroll
+  for (int q = 1; q < 11; q++) p = fma(p, z, c.la[q]);
+  const DD h = dd_fast_sum(sh, sl + sh * z * p);     // ln m / 2
+  const double ph = h.hi * c.l2h;
+  const double pl = fma(h.hi, c.l2l, fma(h.lo, c.l2h, fma(h.hi, c.l2h, -ph)));
+  const DD q = dd_fast_sum(-(double)n, ph);
+  return dd_fast_sum(q.hi, q.lo + pl);
+}
+
+// exp2_dd for |y| < 1022
+__device__ __forceinline__ double exp2_dd_fast(double yh, double yl, const PowSeries& c) {
+  const double n = rint(yh);
+  const double f = yh - n;
+  const double gh = f * c.n2h;
+  const double gl = fma(f, c.n2l, fma(yl, c.n2h, fma(f, c.n2h, -gh)));
+  double q = c.ex[0];
+#pragma unroll
+  for (int s = 1; s < 13; s++) q = fma(q, gh, c.ex[s]);
+  const double u = gh * gh * q;
+  const DD one = dd_fast_sum(1.0, gh);
+  const double r = one.hi + (one.lo + fma(gl, one.hi + u, u));
+  return ldexp(r, (int)n);
+}
+
+// M of one call, capped: t = num / dvds with y = recip(dvds), D = log2 dvds.
+// The bound 0 below takes the NaN of dvds = 0 to the reference's M = 0
+// (krad >= 0 here, so that it changes no other M).
+__device__ __forceinline__ double force_mult_fast(const Const& k, const PowNum& a, double dvds,
+                                                  double y, DD D, const PowSeries& c) {
+  const double t = quot(a.num, dvds, y);
+  const double eps = fma(t, dvds, -a.num) * a.rn;     // rn: log2 e / num
+  const DD d = dd_two_sum(a.L.hi, -D.hi);
+  const DD dl = dd_fast_sum(d.hi, d.lo + ((a.L.lo - D.lo) + eps));
+  const double yh = k.alpharad * dl.hi;
+  const double yl = fma(k.alpharad, dl.lo, fma(k.alpharad, dl.hi, -yh));
+  return fmin(fmax(k.krad * exp2_dd_fast(yh, yl, c), 0.0), 4400.);
 }
 
 PMX_HD void force_mult_pair(const Const& k, double A1, double A2, double dvds,
