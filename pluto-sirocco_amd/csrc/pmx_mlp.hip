@@ -11,7 +11,8 @@
 //                       integrator (the same device code as the wind's
 //                       SplitSource), log-uniform over the training hull
 //   mlp_train_kernel    forward + backward of 16-sample tiles on
-//                       v_mfma_f32_16x16x16_bf16; per-workgroup partial
+//                       v_mfma_f32_16x16x16_bf16, four tiles of four
+//                       wavefronts per workgroup; per-workgroup partial
 //                       gradients (deterministic reduction)
 //   mlp_update_kernel   gradient reduction in a fixed order + Adam (FP32
 //                       master weights) + BF16 copies for the next step
@@ -95,185 +96,213 @@ __global__ void mlp_sample_kernel(Const k, long long n, unsigned long long seed,
 // ---------------------------------------------------------------------
 // training
 // ---------------------------------------------------------------------
-struct alignas(16) TrainLds {
-  unsigned short Xb[16 * 16], XT[16 * 16];
-  float Z1[16 * 64], Z2[16 * 64], Z3[16 * 64];
-  unsigned short H1[16 * 64], H2[16 * 64], H3[16 * 64];
-  unsigned short H1T[64 * 16], H2T[64 * 16];
-  unsigned short dA[16 * 64], dAT[64 * 16];
-  unsigned short dB[16 * 64], dBT[64 * 16];
-  float y[16], t[16], dy[16];
+// Row strides in LDS, padded so that the 16 rows a fragment load touches
+// fall into different banks (a row of 64 BF16 values is one pass over them).
+constexpr int SH = 72;    // [16 samples][64] BF16
+constexpr int ST = 20;    // [64][16 samples] BF16
+constexpr int SV = 68;    // [16 samples][64] FP32
+constexpr int TRAIN_TILES = 4;
+
+struct alignas(16) TrainTile {
+  unsigned short XT[16 * ST];
+  unsigned short H1[16 * SH], H2[16 * SH], H3[16 * SH], H1T[64 * ST], H2T[64 * ST];
+  unsigned short dA[16 * SH], dAT[64 * ST], dB[16 * SH], dBT[64 * ST], dCT[64 * ST];
+  float v1[16 * SV], v2[16 * SV], v3[16 * SV];   // dL/dz of the three layers
+  float g4[64], db[64], loss[16];
 };
 
-// One 64-lane workgroup per block; each runs `tiles` tiles of 16 samples
-// starting at sample `start + blockIdx.x * tiles * 16` (mod n), and writes
+// Forward and backward of a batch.  A workgroup takes TRAIN_TILES tiles of
+// 16 samples from sample `start + blockIdx.x * 64` (mod n) on and writes
 // its summed gradient of  L = sum (y - t)^2 / batch  to partial[block],
 // where t = label / YS is the scaled target.
-__global__ __launch_bounds__(64) void mlp_train_kernel(Weights w, const float* X, const float* Y,
-                                                       long long n, long long start, int tiles,
-                                                       float inv_batch, long long nvalid_limit,
-                                                       float* partial, float* lossp) {
-  __shared__ TrainLds S;
-  const int l = threadIdx.x, r = l & 15, c = l & 15, r0 = (l >> 4) * 4, kq = (l >> 4) * 4;
-  f4 acc1[4], acc2[4][4], acc3[4][4];
+//
+// The network is tiny, so the launch is bound by the length of its
+// dependent chain, not by the matrix cores: 16 wavefronts share a workgroup,
+// one per tile and 16-unit block of a layer, every weight fragment is loaded
+// at the start, and a wavefront keeps its pre-activations and their sigmoids
+// in registers for the backward pass.  The weight gradients chain the tiles
+// in order through the accumulators, 16 wavefronts for the 16 blocks of a
+// 64 x 64 matrix.  Every sum runs in the order of one wavefront taking the
+// tiles one after the other (which took 86 us per 8,192 samples on 128
+// wavefronts), so the gradients are the same to the bit.
+__global__ __launch_bounds__(1024) void mlp_train_kernel(Weights w, const float* X, const float* Y,
+                                                         long long n, long long start,
+                                                         float inv_batch, long long nvalid_limit,
+                                                         float* partial, float* lossp) {
+  __shared__ TrainTile S[TRAIN_TILES];
+  const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = wv >> 2, nt = wv & 3;
+  const int r = l & 15, kq = (l >> 4) * 4, r0 = kq, nn = nt * 16 + r;
+  TrainTile& T = S[tile];
+  // ---- weights of this wavefront's 16 units, and its samples -----------
+  const unsigned short* row = w.W2 + nn * 64 + kq;
+  const int dW3 = (int)(w.W3 - w.W2), dW2T = (int)(w.W2T - w.W2), dW3T = (int)(w.W3T - w.W2);
+  const s4 w1 = frag(w.W1p + nn * 16 + kq);
+  s4 w2[4], w3[4], w2t[4], w3t[4];
 #pragma unroll
-  for (int a = 0; a < 4; a++) {
-    acc1[a] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < 4; b++) acc2[a][b] = acc3[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < 4; q++) {
+    w2[q] = frag(row + q * 16);
+    w3[q] = frag(row + dW3 + q * 16);
+    w3t[q] = frag(row + dW3T + q * 16);
+    w2t[q] = frag(row + dW2T + q * 16);
   }
-  float gb1[4] = {0.f, 0.f, 0.f, 0.f}, gb2[4] = {0.f, 0.f, 0.f, 0.f}, gb3[4] = {0.f, 0.f, 0.f, 0.f};
-  float g4 = 0.f, gb4 = 0.f, loss = 0.f;
-  const long long base = start + (long long)blockIdx.x * tiles * 16;
-  for (int tile = 0; tile < tiles; tile++) {
-    // ---- load 16 samples -------------------------------------------
-    const long long lin = base + tile * 16 + r;   // position inside the batch
-    const long long sidx = lin % n;
-    const float label = Y[sidx];
-    // samples past the batch and unlabelled ones (NaN) carry no loss
-    const bool valid = (lin - start) < nvalid_limit && label == label;
-    float xin[4];
-    load_features(X + 4 * sidx, xin);
+  const float b1 = w.P[OFF_B1 + nn], b2 = w.P[OFF_B2 + nn], b3 = w.P[OFF_B3 + nn];
+  const float w4n = bf2f(w.w4[nn]);
+  const long long lin = start + ((long long)blockIdx.x * TRAIN_TILES + tile) * 16 + r;
+  const long long sidx = lin < n ? lin : lin % n;
+  const float label = Y[sidx];
+  // samples past the batch and unlabelled ones (NaN) carry no loss
+  const bool valid = (lin - start) < nvalid_limit && label == label;
+  float xin[4];
+  load_features(X + 4 * sidx, xin);
+  s4 xa;                       // inputs 4 .. 15 of the padded first layer are 0
 #pragma unroll
-    for (int f = 0; f < 4; f++) {
-      int col = kq + f;
-      float v = (col < 4 && valid) ? xin[col] : 0.f;
-      unsigned short b = f2bf(v);
-      S.Xb[r * 16 + col] = b;
-      S.XT[col * 16 + r] = b;
-    }
-    if (l < 16) {
-      S.t[r] = valid ? label * (1.f / YS) : 0.f;   // the network fits log10(T_f/T_0) / YS
-      S.dy[r] = valid ? 1.f : 0.f;   // validity mask until the loss is known
-    }
-    __syncthreads();
-    // ---- forward ---------------------------------------------------
-    f4 acc[4];
-    dense16<16>(S.Xb, w.W1p, acc, l);
-    epilogue(acc, w.P + OFF_B1, S.Z1, S.H1, S.H1T, l);
-    __syncthreads();
-    dense16<64>(S.H1, w.W2, acc, l);
-    epilogue(acc, w.P + OFF_B2, S.Z2, S.H2, S.H2T, l);
-    __syncthreads();
-    dense16<64>(S.H2, w.W3, acc, l);
-    epilogue(acc, w.P + OFF_B3, S.Z3, S.H3, nullptr, l);
-    __syncthreads();
-    float y = output_unit(S.H3, w, l);
-    if (l < 16) {
-      float m = S.dy[r];
-      float res = (y - S.t[r]) * m;
-      S.y[r] = y;
-      S.dy[r] = 2.f * res * inv_batch;
-      loss += res * res;
-    }
-    __syncthreads();
-    // ---- backward --------------------------------------------------
-    {
-      float s4sum = 0.f, db = 0.f;
+  for (int f = 0; f < 4; f++) xa[f] = (short)f2bf((kq == 0 && valid) ? xin[f] : 0.f);
+  if (nt == 0) {
 #pragma unroll
-      for (int s = 0; s < 16; s++) {
-        s4sum += bf2f(S.H3[s * 64 + l]) * S.dy[s];
-        db += S.dy[s];
-      }
-      g4 += s4sum;
-      gb4 += db;
-    }
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int nn = nt * 16 + c;
-      const float wv = bf2f(w.w4[nn]);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int s = r0 + i;
-        float v = S.dy[s] * wv * dsilu(S.Z3[s * 64 + nn]);
-        unsigned short b = f2bf(v);
-        S.dA[s * 64 + nn] = b;
-        S.dAT[nn * 16 + s] = b;
-        gb3[nt] += v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-      s4 a = frag(S.dAT + (mt * 16 + r) * 16 + kq);
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        acc3[mt][nt] = mma(a, frag(S.H2T + (nt * 16 + r) * 16 + kq), acc3[mt][nt]);
-    }
-    dense16<64>(S.dA, w.W3T, acc, l);   // dH2 = dZ3 W3
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int nn = nt * 16 + c;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int s = r0 + i;
-        float v = acc[nt][i] * dsilu(S.Z2[s * 64 + nn]);
-        unsigned short b = f2bf(v);
-        S.dB[s * 64 + nn] = b;
-        S.dBT[nn * 16 + s] = b;
-        gb2[nt] += v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-      s4 a = frag(S.dBT + (mt * 16 + r) * 16 + kq);
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++)
-        acc2[mt][nt] = mma(a, frag(S.H1T + (nt * 16 + r) * 16 + kq), acc2[mt][nt]);
-    }
-    dense16<64>(S.dB, w.W2T, acc, l);   // dH1 = dZ2 W2
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int nn = nt * 16 + c;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int s = r0 + i;
-        float v = acc[nt][i] * dsilu(S.Z1[s * 64 + nn]);
-        S.dAT[nn * 16 + s] = f2bf(v);
-        gb1[nt] += v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++)
-      acc1[mt] = mma(frag(S.dAT + (mt * 16 + r) * 16 + kq), frag(S.XT + r * 16 + kq), acc1[mt]);
-    __syncthreads();
+    for (int f = 0; f < 4; f++) T.XT[(kq + f) * ST + r] = (unsigned short)xa[f];
   }
-  // ---- partial gradient of this workgroup ---------------------------
-  float* out = partial + (long long)blockIdx.x * NPP;
-#pragma unroll
-  for (int mt = 0; mt < 4; mt++)
+  // z, sigmoid(z) of the wavefront's 4 values per layer
+  float z1[4], s1[4], z2[4], s2[4], z3[4], s3[4];
+  auto activate = [&](f4 acc, float b, float* z, float* sg, unsigned short* H,
+                      unsigned short* HT) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int m = mt * 16 + r0 + i;
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++) {
-        out[OFF_W3 + m * 64 + nt * 16 + c] = acc3[mt][nt][i];
-        out[OFF_W2 + m * 64 + nt * 16 + c] = acc2[mt][nt][i];
-      }
-      if (c < 4) out[OFF_W1 + m * 4 + c] = acc1[mt][i];
+      z[i] = acc[i] + b;
+      sg[i] = sigm(z[i]);
+      const unsigned short hb = f2bf(z[i] * sg[i]);
+      H[(r0 + i) * SH + nn] = hb;
+      if (HT) HT[nn * ST + r0 + i] = hb;
     }
+  };
+  auto dense = [&](const unsigned short* in, const s4* wf) {
+    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++) {
-    float a1 = gb1[nt], a2 = gb2[nt], a3 = gb3[nt];
-    a1 += __shfl_xor(a1, 16); a1 += __shfl_xor(a1, 32);
-    a2 += __shfl_xor(a2, 16); a2 += __shfl_xor(a2, 32);
-    a3 += __shfl_xor(a3, 16); a3 += __shfl_xor(a3, 32);
-    if (l < 16) {
-      out[OFF_B1 + nt * 16 + l] = a1;
-      out[OFF_B2 + nt * 16 + l] = a2;
-      out[OFF_B3 + nt * 16 + l] = a3;
-    }
+    for (int q = 0; q < 4; q++) acc = mma(frag(in + r * SH + q * 16 + kq), wf[q], acc);
+    return acc;
+  };
+  // ---- forward ---------------------------------------------------------
+  activate(mma(xa, w1, f4{0.f, 0.f, 0.f, 0.f}), b1, z1, s1, T.H1, T.H1T);
+  __syncthreads();
+  activate(dense(T.H1, w2), b2, z2, s2, T.H2, T.H2T);
+  __syncthreads();
+  activate(dense(T.H2, w3), b3, z3, s3, T.H3, nullptr);
+  __syncthreads();
+  // y of sample r, in every lane of its column and every wavefront
+  float y;
+  {
+    const int k0 = (l >> 4) * 16;
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) sum += bf2f(T.H3[r * SH + k0 + k]) * bf2f(w.w4[k0 + k]);
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    y = sum + w.P[OFF_B4];
   }
-  out[OFF_W4 + l] = g4;
-  loss += __shfl_xor(loss, 1); loss += __shfl_xor(loss, 2); loss += __shfl_xor(loss, 4);
-  loss += __shfl_xor(loss, 8);
-  if (l == 0) {
-    out[OFF_B4] = gb4;
-    lossp[blockIdx.x] = loss;
+  const float res = (y - (valid ? label * (1.f / YS) : 0.f)) * (valid ? 1.f : 0.f);
+  const float dy = 2.f * res * inv_batch;
+  if (nt == 0) {
+    if (l < 16) T.loss[l] = 0.f + res * res;
+    float s4sum = 0.f, db = 0.f;
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      const float d = __shfl(dy, s);
+      s4sum += bf2f(T.H3[s * SH + l]) * d;
+      db += d;
+    }
+    T.g4[l] = s4sum;
+    T.db[l] = db;
+  }
+  // ---- backward --------------------------------------------------------
+  // dL/dz = d silu'(z), kept in FP32 for the biases
+  auto back = [&](const float* d, const float* z, const float* sg, float* v,
+                  unsigned short* D, unsigned short* DT) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float g = d[i] * (sg[i] * (1.f + z[i] * (1.f - sg[i])));
+      const unsigned short b = f2bf(g);
+      if (D) D[(r0 + i) * SH + nn] = b;
+      DT[nn * ST + r0 + i] = b;
+      v[(r0 + i) * SV + nn] = g;
+    }
+  };
+  // block (mt, nt) of a weight gradient dZ^T H, the tiles in order
+  const int mt = wv >> 2;
+  float d[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) d[i] = __shfl(dy, r0 + i) * w4n;
+  back(d, z3, s3, T.v3, T.dA, T.dAT);
+  __syncthreads();
+  f4 acc3 = f4{0.f, 0.f, 0.f, 0.f}, acc2 = acc3, acc1 = acc3;
+  {
+    const f4 a = dense(T.dA, w3t);   // dH2 = dZ3 W3
+#pragma unroll
+    for (int q = 0; q < TRAIN_TILES; q++)
+      acc3 = mma(frag(S[q].dAT + (mt * 16 + r) * ST + kq), frag(S[q].H2T + nn * ST + kq), acc3);
+#pragma unroll
+    for (int i = 0; i < 4; i++) d[i] = a[i];
+    back(d, z2, s2, T.v2, T.dB, T.dBT);
+  }
+  __syncthreads();
+  {
+    const f4 a = dense(T.dB, w2t);   // dH1 = dZ2 W2
+#pragma unroll
+    for (int q = 0; q < TRAIN_TILES; q++)
+      acc2 = mma(frag(S[q].dBT + (mt * 16 + r) * ST + kq), frag(S[q].H1T + nn * ST + kq), acc2);
+#pragma unroll
+    for (int i = 0; i < 4; i++) d[i] = a[i];
+    back(d, z1, s1, T.v1, nullptr, T.dCT);
+  }
+  __syncthreads();
+  // ---- partial gradient of this workgroup ------------------------------
+  float* out = partial + (long long)blockIdx.x * NPP;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int m = mt * 16 + r0 + i;
+    out[OFF_W3 + m * 64 + nn] = acc3[i];
+    out[OFF_W2 + m * 64 + nn] = acc2[i];
+  }
+  if (wv < 12) {
+    // biases: layer wv / 4, units of block nt, summed over tiles and rows
+    const int layer = wv >> 2;
+    float g = 0.f;
+#pragma unroll
+    for (int q = 0; q < TRAIN_TILES; q++) {
+      const float* v = layer == 0 ? S[q].v1 : (layer == 1 ? S[q].v2 : S[q].v3);
+#pragma unroll
+      for (int i = 0; i < 4; i++) g += v[(r0 + i) * SV + nn];
+    }
+    g += __shfl_xor(g, 16);
+    g += __shfl_xor(g, 32);
+    if (l < 16) out[(layer == 0 ? OFF_B1 : (layer == 1 ? OFF_B2 : OFF_B3)) + nn] = g;
+  } else {
+    // first layer: block nt of its 64 rows
+#pragma unroll
+    for (int q = 0; q < TRAIN_TILES; q++)
+      acc1 = mma(frag(S[q].dCT + nn * ST + kq), frag(S[q].XT + r * ST + kq), acc1);
+    if (r < 4) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) out[OFF_W1 + (nt * 16 + r0 + i) * 4 + r] = acc1[i];
+    }
+    if (nt == 3) {
+      float g4 = 0.f, gb4 = 0.f, loss = 0.f;
+#pragma unroll
+      for (int q = 0; q < TRAIN_TILES; q++) {
+        g4 += S[q].g4[l];
+        gb4 += S[q].db[l];
+        loss += S[q].loss[r];
+      }
+      out[OFF_W4 + l] = g4;
+      loss += __shfl_xor(loss, 1); loss += __shfl_xor(loss, 2); loss += __shfl_xor(loss, 4);
+      loss += __shfl_xor(loss, 8);
+      if (l == 0) {
+        out[OFF_B4] = gb4;
+        lossp[blockIdx.x] = loss;
+      }
+    }
   }
 }
+static_assert(sizeof(TrainTile) * TRAIN_TILES <= 160 * 1024, "LDS of a compute unit");
 
 // Writes the BF16 operand copies of parameter p.
 __device__ __forceinline__ void write_bf16(const Weights& w, int p, float v) {
@@ -295,22 +324,40 @@ __device__ __forceinline__ void write_bf16(const Weights& w, int p, float v) {
   }
 }
 
+// p[0] + p[stride] + ... over n values in that order, 32 loads at a time
+// (the sum is a chain of additions; its loads need not be).
+__device__ __forceinline__ float sum_in_order(const float* p, long long stride, int n) {
+  float s = 0.f;
+  int q = 0;
+  for (; q + 32 <= n; q += 32) {
+    float v[32];
+#pragma unroll
+    for (int u = 0; u < 32; u++) v[u] = p[(q + u) * stride];
+#pragma unroll
+    for (int u = 0; u < 32; u++) s += v[u];
+  }
+  for (; q < n; q++) s += p[q * stride];
+  return s;
+}
+
 // Sum of the partial gradients in block order, then either the gradient
 // is stored (grad != nullptr) or one Adam step is applied (FP32 master
-// weights) and the BF16 copies refreshed.  Thread 0 also records the
-// summed loss of the step.
-__global__ void mlp_update_kernel(Weights w, float* m1, float* m2, const float* partial,
-                                  int nwg, const float* lossp, float* loss_out, float lr,
-                                  float bc1, float bc2, float* grad) {
+// weights) and the BF16 copies refreshed.  The last workgroup records the
+// summed loss of the step.  Small workgroups: the launch is bound by the
+// latency of the partials' loads (34 us with 256 threads and one load at a
+// time for the 128 partials of 8,192 samples).
+__global__ __launch_bounds__(64) void mlp_update_kernel(Weights w, float* m1, float* m2,
+                                                        const float* partial, int nwg,
+                                                        const float* lossp, float* loss_out,
+                                                        float lr, float bc1, float bc2,
+                                                        float* grad) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p == 0 && loss_out) {
-    float s = 0.f;
-    for (int q = 0; q < nwg; q++) s += lossp[q];
-    *loss_out = s;
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x == 0 && loss_out) *loss_out = sum_in_order(lossp, 1, nwg);
+    return;
   }
   if (p >= NP) return;
-  float g = 0.f;
-  for (int q = 0; q < nwg; q++) g += partial[(long long)q * NPP + p];
+  const float g = sum_in_order(partial + p, NPP, nwg);
   if (grad) {
     grad[p] = g;
     return;
@@ -325,6 +372,7 @@ __global__ void mlp_update_kernel(Weights w, float* m1, float* m2, const float* 
   P[p] = np;
   write_bf16(w, p, np);
 }
+constexpr int UPDATE_BLOCKS = (NP + 63) / 64 + 1;
 
 __global__ void mlp_sync_kernel(Weights w) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -855,14 +903,13 @@ int pmx_mlp_get_dataset(pmx_mlp* m, float* X, float* Y, int* nev, double* aux, l
 // Loss and gradient of the first `count` dataset samples (one batch).
 int pmx_mlp_loss_grad(pmx_mlp* m, long long count, float* loss, float* grad) {
   if (!m || count <= 0 || count > m->n || !grad) { set_error("bad argument"); return -1; }
-  const int tiles = 4;
-  const int nwg = (int)((count + 16 * tiles - 1) / (16 * tiles));
+  const int nwg = (int)((count + 16 * TRAIN_TILES - 1) / (16 * TRAIN_TILES));
   if (ensure_partials(m, nwg)) return -1;
   float* dgrad = nullptr;
   PMX_HIP_CHECK(hipMalloc(&dgrad, sizeof(float) * (NP + 1)));
-  hipLaunchKernelGGL(mlp_train_kernel, dim3(nwg), dim3(64), 0, m->stream, m->w, m->X, m->Y,
-                     m->n, 0ll, tiles, 1.f / (float)count, count, m->partial, m->lossp);
-  hipLaunchKernelGGL(mlp_update_kernel, dim3((NP + 255) / 256), dim3(256), 0, m->stream, m->w,
+  hipLaunchKernelGGL(mlp_train_kernel, dim3(nwg), dim3(1024), 0, m->stream, m->w, m->X, m->Y,
+                     m->n, 0ll, 1.f / (float)count, count, m->partial, m->lossp);
+  hipLaunchKernelGGL(mlp_update_kernel, dim3(UPDATE_BLOCKS), dim3(64), 0, m->stream, m->w,
                      m->m1, m->m2, m->partial, nwg, m->lossp, dgrad + NP, 0.f, 1.f, 1.f, dgrad);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(grad, dgrad, sizeof(float) * NP, hipMemcpyDeviceToHost, m->stream);
@@ -880,8 +927,7 @@ int pmx_mlp_loss_grad(pmx_mlp* m, long long count, float* loss, float* grad) {
 // loss_hist (optional, `steps` entries) receives each step's mean loss.
 int pmx_mlp_train(pmx_mlp* m, int steps, int batch, float lr0, float lr1, float* loss_hist) {
   if (!m || steps <= 0 || batch <= 0 || batch % 64 || !m->X) { set_error("bad argument"); return -1; }
-  const int tiles = 4;
-  const int nwg = batch / (16 * tiles);
+  const int nwg = batch / (16 * TRAIN_TILES);
   if (ensure_partials(m, nwg)) return -1;
   float* dl = nullptr;
   PMX_HIP_CHECK(hipMalloc(&dl, sizeof(float) * steps));
@@ -892,10 +938,10 @@ int pmx_mlp_train(pmx_mlp* m, int steps, int batch, float lr0, float lr1, float*
     const float lr = (float)(lr1 + 0.5 * (lr0 - lr1) * (1.0 + cos(3.14159265358979 * ph)));
     const float bc1 = (float)(1.0 - pow(0.9, (double)m->adam_t));
     const float bc2 = (float)(1.0 - pow(0.999, (double)m->adam_t));
-    hipLaunchKernelGGL(mlp_train_kernel, dim3(nwg), dim3(64), 0, m->stream, m->w, m->X, m->Y,
-                       m->n, start, tiles, 1.f / (float)batch, (long long)batch, m->partial,
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(nwg), dim3(1024), 0, m->stream, m->w, m->X, m->Y,
+                       m->n, start, 1.f / (float)batch, (long long)batch, m->partial,
                        m->lossp);
-    hipLaunchKernelGGL(mlp_update_kernel, dim3((NP + 255) / 256), dim3(256), 0, m->stream,
+    hipLaunchKernelGGL(mlp_update_kernel, dim3(UPDATE_BLOCKS), dim3(64), 0, m->stream,
                        m->w, m->m1, m->m2, m->partial, nwg, m->lossp, dl + s, lr, bc1, bc2,
                        (float*)nullptr);
     start = (start + batch) % m->n;
