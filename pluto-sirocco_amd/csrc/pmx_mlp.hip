@@ -51,7 +51,7 @@ __device__ __forceinline__ double unif(unsigned long long seed, unsigned long lo
 // parameter and dt / t_cool drawn log-uniformly over the hull, integrated
 // over dt by the plain integrator (g_time > 3, so Radiat takes xi and T_r
 // from the SIROCCO arrays; tracer 1).
-__global__ void mlp_sample_kernel(Const k, long long n, unsigned long long seed, float* X,
+__global__ __launch_bounds__(128) void mlp_sample_kernel(Const k, long long n, unsigned long long seed, float* X,
                                   float* Y, int* nev, double* aux) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n) return;
@@ -65,6 +65,7 @@ __global__ void mlp_sample_kernel(Const k, long long n, unsigned long long seed,
   R.rho = rho; R.trc = 1.0; R.x1 = 1.0; R.xi_s = pow(10.0, lx); R.tr_s = k.t_x; R.t = 5.0;
   wind::load_pre(nullptr, 0, 0, R.pre);
   R.nev = 0;
+  wind::rad_prepare(k, R);
   double T0 = p0 / rho * k.KELVIN * k.mu;
   double E0 = p0 / (k.gamma - 1.0);
   double k1 = wind::radiat(k, R, E0);
@@ -450,6 +451,7 @@ __device__ __forceinline__ RadCell cell_state(const CoolArgs& a, long long cell)
   wind::load_pre(a.pre, a.sv, cell, R.pre);
   R.t = a.s->t;
   R.nev = 0;
+  wind::rad_prepare(a.k, R);
   return R;
 }
 

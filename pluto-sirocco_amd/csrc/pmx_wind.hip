@@ -1057,6 +1057,7 @@ __global__ __launch_bounds__(128) void wind_cool_kernel(CoolArgs a, unsigned lon
       load_pre(a.pre, a.sv, cell, R.pre);
       R.t = t;
       R.nev = 0;
+      rad_prepare(a.k, R);
       pn = plain_cell(a.k, R, p, dt, cand, bad);
       ncalls = R.nev;
     }

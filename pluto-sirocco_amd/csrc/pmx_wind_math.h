@@ -746,28 +746,75 @@ struct RadCell {
   double pre[5];   // comp_h, comp_c, xray_h, brem_c, line_c (cooling_source.c:101-105)
   double t;        // g_time
   mutable int nev; // Radiat() evaluations so far (cost accounting)
+  // set by rad_prepare: what Radiat() forms from the above alone
+  double nH, xi, tx, sqxi, sqsqxi;
+  double rrho, rsqxi;   // recip(rho), recip(sqxi)
+  bool moderate;        // rho and xi within radiat<true>'s range
 };
 
+PMX_HD bool in_range(double x, double lo, double hi) { return x >= lo && x <= hi; }
+
+PMX_HD void rad_prepare(const Const& k, RadCell& R) {
+  const double rho = R.rho * k.UD;
+  R.nH = rho / (1.43 * C_mp);
+  const double r = R.x1 * k.UL;
+  if (R.t < 3.0) { R.xi = k.lx / R.nH / r / r; R.tx = k.t_x; }
+  else { R.xi = R.xi_s; R.tx = R.tr_s; }
+  R.sqxi = sqrt(R.xi);
+  R.sqsqxi = pow(R.xi, 0.25);
+  R.moderate = in_range(R.rho, 0x1p-200, 0x1p200) && in_range(R.xi, 0x1p-200, 0x1p200) &&
+               in_range(k.KELVIN * k.mu, 0x1p-100, 0x1p100);
+  R.rrho = recip(R.rho);
+  R.rsqxi = recip(R.sqxi);
+}
+
+// Largest energy of radiat<true>; a cell that exceeds it is done again with
+// the general operations.
+constexpr double RAD_E_MAX = 0x1p300;
+
+// a / b, by the moderate quotient where MOD
+template <bool MOD>
+PMX_HD double mdiv(double a, double b) {
+  if constexpr (MOD) return quot(a, b, recip(b));
+  else return a / b;
+}
+
 // Radiat(): returns the RHOE rate; may floor *E like the reference.
-PMX_HD double radiat(const Const& k, const RadCell& R, double& E) {
+//
+// A cell whose cooling takes 10^5 evaluations in a row holds up its launch,
+// and each is one long dependent chain, so MOD leaves out of its divisions
+// and its root what moderate operands do not need and shares the
+// reciprocals (rho's and sqrt(xi)'s from rad_prepare, T's three times):
+// about 115 instructions instead of 180, the same bits.  For a cell with
+// R.moderate and E <= RAD_E_MAX (`over` tells): then T >= 1e4 K from here on
+// bounds every other operand.
+template <bool MOD = false>
+PMX_HD double radiat(const Const& k, const RadCell& R, double& E, bool& over) {
   const double minT = 1.e4;
   R.nev++;
   double prs = E * (k.gamma - 1.0);
   if (prs < 0.0) { prs = 1.e-12; E = prs / (k.gamma - 1.0); }
-  double T = prs / R.rho * k.KELVIN * k.mu;
+  if (MOD) over = over | !(E <= RAD_E_MAX);
+  double T = (MOD ? quot(prs, R.rho, R.rrho) : prs / R.rho) * k.KELVIN * k.mu;
   if (T < minT) return 0.0;
-  double rho = R.rho * k.UD, nH = rho / (1.43 * C_mp);
-  double r = R.x1 * k.UL, xi, tx;
-  if (R.t < 3.0) { xi = k.lx / nH / r / r; tx = k.t_x; }
-  else { xi = R.xi_s; tx = R.tr_s; }
-  double sqT = sqrt(T), sqxi = sqrt(xi), sqsqxi = pow(xi, 0.25);
+  const double nH = R.nH, xi = R.xi, tx = R.tx, sqxi = R.sqxi, sqsqxi = R.sqsqxi;
+  double sqT, rT = 0.0, rsqT = 0.0;
+  if constexpr (MOD) {
+    sqT = sqrt_mod(T, rsqT);
+    rsqT = fma(rsqT, fma(-sqT, rsqT, 1.0), rsqT);
+    rT = recip(T);
+  } else {
+    sqT = sqrt(T);
+  }
+  auto by_T = [&](double x) { return MOD ? quot(x, T, rT) : x / T; };
   double ne = 1.21 * nH;
   // cv_idl/radiat.c:118-123
   double comp_heat = R.pre[0] * (8.9e-36 * xi * tx);
   double comp_cool = R.pre[1] * (8.9e-36 * xi * (4.0 * T));
-  double xray_heat = R.pre[2] * (1.5e-21 * (sqsqxi / sqT));
-  double line_cool = R.pre[4] * ((1e-16 * exp(-1.3e5 / T) / sqxi / T) +
-                                 fmin(fmin(1e-24, 5e-27 * sqT), 1.5e-17 / T));
+  double xray_heat = R.pre[2] * (1.5e-21 * (MOD ? quot(sqsqxi, sqT, rsqT) : sqsqxi / sqT));
+  const double le = 1e-16 * exp(by_T(-1.3e5));
+  double line_cool = R.pre[4] * (by_T(MOD ? quot(le, sqxi, R.rsqxi) : le / sqxi) +
+                                 fmin(fmin(1e-24, 5e-27 * sqT), by_T(1.5e-17)));
   double brem_cool = R.pre[3] * (3.3e-27 * sqT);
   double lambda = nH * (ne * comp_heat + nH * xray_heat - ne * comp_cool - ne * line_cool -
                         ne * brem_cool);
@@ -776,21 +823,26 @@ PMX_HD double radiat(const Const& k, const RadCell& R, double& E) {
   // 2^-54 (y > 38): from T/minT >= 1.4 on (y >= 56.7, 1/cosh(y) < 5e-25,
   // far beyond any last-bit error of pow or cosh) the factor is 1.0 and
   // the two calls are skipped, bit for bit the same result
-  const double tr = T / minT;
-  if (!(tr >= 1.4)) rhs *= 1.0 - 1.0 / cosh(pow(tr, 12));
+  if (!(T >= 1.4 * minT)) rhs *= 1.0 - 1.0 / cosh(pow(T / minT, 12));
   return rhs;
 }
 
+PMX_HD double radiat(const Const& k, const RadCell& R, double& E) {
+  bool over = false;
+  return radiat<false>(k, R, E, over);
+}
+
 // SolveODE_RKF12: returns err, writes the 2nd-order result.
+template <bool MOD>
 PMX_HD double rkf12(const Const& k, const RadCell& R, double E0, double k1,
-                                        double& E2nd, double dt) {
+                                        double& E2nd, double dt, bool& over) {
   double E1 = E0 + 0.5 * dt * k1;
-  double k2 = radiat(k, R, E1);
+  double k2 = radiat<MOD>(k, R, E1, over);
   E2nd = E0 + dt * k2;
   double E1st = E0 + dt * k1;
   double vscal = fabs(E0) + dt * fabs(k1);
   double err = 0.0;
-  double scrh = fabs(E2nd - E1st) / fabs(vscal);
+  double scrh = mdiv<MOD>(fabs(E2nd - E1st), fabs(vscal));
   return dmax(err, scrh);
 }
 
@@ -798,8 +850,9 @@ PMX_HD double rkf12(const Const& k, const RadCell& R, double E0, double k1,
 // proposed next step.  E0 and k1 belong to the caller and are not
 // changed.  `nsub` counts accepted sub-steps (the reference aborts the
 // run past 1000; here the caller sees the count and flags the cell).
+template <bool MOD>
 PMX_HD_NOINLINE double ck45(const Const& k, const RadCell& R, double E0, double k1, double& E5th,
-                       double dt, double tol, int& nsub) {
+                       double dt, double tol, int& nsub, bool& over) {
   const double c1 = 37.0 / 378.0, c2 = 0.0, c3 = 250.0 / 621.0, c4 = 125.0 / 594.0, c5 = 0.0,
                c6 = 512.0 / 1771.0;
   const double cs1 = 2825.0 / 27648.0, cs2 = 0.0, cs3 = 18575.0 / 48384.0,
@@ -814,20 +867,20 @@ PMX_HD_NOINLINE double ck45(const Const& k, const RadCell& R, double E0, double 
     if (iter >= CK45_ITER_MAX) { ksub = 1001; break; }
     double E1, k2, k3, k4, k5, k6;
     E1 = E0 + dt * b21 * k1;
-    k2 = radiat(k, R, E1);
+    k2 = radiat<MOD>(k, R, E1, over);
     E1 = E0 + dt * (b31 * k1 + b32 * k2);
-    k3 = radiat(k, R, E1);
+    k3 = radiat<MOD>(k, R, E1, over);
     E1 = E0 + dt * (b41 * k1 + b42 * k2 + b43 * k3);
-    k4 = radiat(k, R, E1);
+    k4 = radiat<MOD>(k, R, E1, over);
     E1 = E0 + dt * (b51 * k1 + b52 * k2 + b53 * k3 + b54 * k4);
-    k5 = radiat(k, R, E1);
+    k5 = radiat<MOD>(k, R, E1, over);
     E1 = E0 + dt * (b61 * k1 + b62 * k2 + b63 * k3 + b64 * k4 + b65 * k5);
-    k6 = radiat(k, R, E1);
+    k6 = radiat<MOD>(k, R, E1, over);
     E5th = E0 + dt * (c1 * k1 + c2 * k2 + c3 * k3 + c4 * k4 + c5 * k5 + c6 * k6);
     double E4th = E0 + dt * (cs1 * k1 + cs2 * k2 + cs3 * k3 + cs4 * k4 + cs5 * k5 + cs6 * k6);
     double vscal = fabs(E0) + dt * fabs(k1);
     double err = 0.0;
-    double scrh = fabs(E5th - E4th) / fabs(vscal);
+    double scrh = mdiv<MOD>(fabs(E5th - E4th), fabs(vscal));
     err = dmax(err, scrh);
     err /= tol;
     if (err < 1.0) {
@@ -840,7 +893,7 @@ PMX_HD_NOINLINE double ck45(const Const& k, const RadCell& R, double E0, double 
       if (fabs(t / tend - 1.0) < 1.e-9) break;
       if (dt > (tend - t)) dt = tend - t;
       E0 = E5th;
-      k1 = radiat(k, R, E0);
+      k1 = radiat<MOD>(k, R, E0, over);
       if (ksub > 1000) break;
     } else {
       double dt_shrink = 0.9 * dt * pow(err, -0.25);
@@ -867,18 +920,17 @@ PMX_HD double finish_cell(const Const& k, const RadCell& R, double p, double E1,
   return prs;
 }
 
-// One cell of CoolingSource: returns the new pressure and the cell's
-// dt * maxCoolingRate / |dp/p| candidate for dt_cool.
-// plain_cell_from: the same from E0 and k1 = Radiat(E0) already formed
-// (E0 as Radiat left it), for a caller that has evaluated the first rate.
-PMX_HD double plain_cell_from(const Const& k, const RadCell& R, double p, double dt, double E0,
-                              double k1, double& dt_cool_cell, int& bad) {
+// One cell of CoolingSource from E0 and k1 = Radiat(E0) (E0 as Radiat left
+// it): the integrated energy.
+template <bool MOD>
+PMX_HD double integrate_cell(const Const& k, const RadCell& R, double dt, double E0, double k1,
+                             int& bad, bool& over) {
   const double min_tol = 2.e-5;
   double E1 = E0;
   int stiff = (fabs(k1) > 0.5 / dt ? 1 : 0);
   double err = 0.0;
   if (!stiff) {
-    err = rkf12(k, R, E0, k1, E1, dt);
+    err = rkf12<MOD>(k, R, E0, k1, E1, dt, over);
     err /= min_tol;
   }
   if (stiff || err > 1.0) {
@@ -888,15 +940,37 @@ PMX_HD double plain_cell_from(const Const& k, const RadCell& R, double p, double
       if (++outer > SUBSTEP_MAX) { bad = 1; break; }
       if ((t1 + dt1) >= dt) { dt1 = dt - t1; done = 1; }
       int nsub = 0;
-      double dts = ck45(k, R, E0, k1, E1, dt1, min_tol, nsub);
+      double dts = ck45<MOD>(k, R, E0, k1, E1, dt1, min_tol, nsub, over);
       if (nsub > 1000) bad = 1;
       t1 += dt1;
       dt1 = dts;
       if (done) break;
       E0 = E1;
-      k1 = radiat(k, R, E0);
+      k1 = radiat<MOD>(k, R, E0, over);
     } while (!done);
   }
+  return E1;
+}
+
+// One cell of CoolingSource: returns the new pressure and the cell's
+// dt * maxCoolingRate / |dp/p| candidate for dt_cool, from a first rate
+// already formed.  A cell of moderate state takes the short operations, and
+// the general ones again if an energy left their range on the way.
+PMX_HD double plain_cell_from(const Const& k, const RadCell& R, double p, double dt, double E0,
+                              double k1, double& dt_cool_cell, int& bad) {
+  const int nev = R.nev;
+  bool general = !(R.moderate && in_range(E0, 0x1p-300, RAD_E_MAX) &&
+                   in_range(dt, 0x1p-300, 0x1p300));
+  double E1 = E0;
+  int b = 0;
+  if (!general) E1 = integrate_cell<true>(k, R, dt, E0, k1, b, general);
+  if (general) {
+    R.nev = nev;
+    b = 0;
+    bool over = false;
+    E1 = integrate_cell<false>(k, R, dt, E0, k1, b, over);
+  }
+  bad |= b;
   return finish_cell(k, R, p, E1, dt, dt_cool_cell);
 }
 
