@@ -16,31 +16,6 @@ namespace pmx {
 static thread_local std::string g_err;
 void set_error(const std::string& msg) { g_err = msg; }
 
-struct DevScalars {
-  double t;                      // g_time
-  double dt;                     // g_dt of the step being taken
-  double inv_dt_hyp;             // Dts->invDt_hyp of the last step
-  double tstop;                  // runtime.tstop
-  double dt_uncut;               // the dt a cut to tstop replaced
-  int err;                       // cons->prim flags of the step under way
-  int step_err;                  // cons->prim flags of the last completed step
-  int halt;                      // PMX_FLAG_DT_TOO_SMALL / PMX_FLAG_TSTOP once set (sticky):
-                                 // later main-loop steps are no-ops
-  int last;                      // the next step is the last one (dt clamped to tstop - t)
-  unsigned long long cdt_red[RED_SLOTS * RED_STRIDE];   // stage-1 C_dt maxima, spread
-                                                        // (words red_index(k), 0 = none)
-};
-
-// Src/main.c:226-229: the step that would reach tstop (to 1e-8 relative)
-// is the last one, and its dt is cut to land on tstop.
-__host__ __device__ inline void clamp_last_step(DevScalars& s) {
-  if ((s.t + s.dt) >= s.tstop * (1.0 - 1.e-8)) {
-    s.dt_uncut = s.dt;
-    s.dt = (s.tstop - s.t);
-    s.last = 1;
-  }
-}
-
 // dt/dx for every cell and direction, and reset of the step reductions.
 // A main-loop step (dt_override null) does nothing once the run has halted.
 __global__ void prep_kernel(DevScalars* s, const double* dx, double* dtdx, int ntot,
@@ -56,68 +31,44 @@ __global__ void prep_kernel(DevScalars* s, const double* dx, double* dtdx, int n
   }
 }
 
-// Src/update_stage.c:389-394 then Src/main.c:596-697 (NextTimeStep, no
-// parabolic terms, no cooling) and the time update of main.c:296.  In the
-// main loop (loop != 0) a halted run does nothing; NextTimeStep's "dt is
-// too small" quit (main.c:672-683) halts it, and so does the end of the
-// step that reached tstop; otherwise the next step's dt is cut to land on
-// tstop when it would pass it (main.c:226-229).  One thread.  Returns
-// whether the run goes on.
-__device__ bool finish_step(DevScalars* s, int ndim, double cfl, double cfl_max_var,
-                            double first_dt, int loop, const double* inv_in) {
-  if (loop && s->halt) return false;
-  double inv = inv_in ? *inv_in : 0.0;   // Dts->invDt_hyp the stage-1 maximum folds into
-  unsigned long long m = 0ull;   // non-negative doubles order like their bit patterns
-#pragma unroll
-  for (int k = 0; k < RED_SLOTS; k++) {
-    const unsigned long long v = s->cdt_red[red_index(k)];
-    m = v > m ? v : m;
-  }
-  double c = __longlong_as_double((long long)m);
-  inv = dmax(inv, c);
-  inv /= (double)ndim;
-  s->inv_dt_hyp = inv;
-  s->step_err = s->err;
-  s->err = 0;
-  double dt = s->dt;
-  s->t += dt;
-  double dt_hyp = 1.0 / inv;
-  dt_hyp *= cfl;
-  double dtnext = dt_hyp;
-  dtnext = dmin(dtnext, cfl_max_var * dt);
-  if (cfl_max_var != 1.0) s->dt = dtnext;
-  if (!loop) return false;
-  if (dtnext < first_dt * 1.e-9) s->halt |= PMX_FLAG_DT_TOO_SMALL;   // main.c:672-683
-  if (s->last) {
-    s->halt |= PMX_FLAG_TSTOP;
-    s->last = 0;
-  } else {
-    DevScalars q = *s;
-    clamp_last_step(q);
-    s->dt = q.dt;
-    s->dt_uncut = q.dt_uncut;
-    s->last = q.last;
-  }
-  return !s->halt;
-}
-
-// finish_step, then, in the main loop while the run goes on, what
+// The end of a step taken through the dt/dx table (3-D, or an explicit
+// step): end_step, then, in the main loop while the run goes on, what
 // prep_kernel would do for the next step: dt/dx with the next dt and the
 // cleared C_dt slots (the next step's own prep launch is then left out).
-__global__ __launch_bounds__(256) void finish_kernel(DevScalars* s, int ndim, double cfl,
-                                                     double cfl_max_var, double first_dt,
-                                                     int loop, const double* inv_in,
-                                                     const double* dx, double* dtdx, int ntot) {
+__global__ __launch_bounds__(256) void finish_kernel(DevScalars* s, StepRule rule, int loop,
+                                                     const double* inv_in, const double* dx,
+                                                     double* dtdx, int ntot) {
   __shared__ int go;
   __shared__ double dt_next;
+  StepState q = *s;
+  const unsigned long long m = fold_cdt(s);
+  __syncthreads();                     // every thread has read before one writes
+  if (loop && q.halt) return;
   if (threadIdx.x == 0) {
-    go = finish_step(s, ndim, cfl, cfl_max_var, first_dt, loop, inv_in) ? 1 : 0;
-    dt_next = s->dt;
+    end_step(q, m, rule, loop, inv_in ? *inv_in : 0.0);
+    static_cast<StepState&>(*s) = q;
+    go = loop && !q.halt;
+    dt_next = q.dt;
   }
   __syncthreads();
   if (!go) return;
   for (int q = threadIdx.x; q < ntot; q += blockDim.x) dtdx[q] = dt_next / dx[q];
   if (threadIdx.x < RED_SLOTS) s->cdt_red[red_index(threadIdx.x)] = 0ull;
+}
+
+// The end of a 2-D main-loop run: end_step on the last step's state
+// s[which], the result in s[0], the reductions of both states cleared.
+__global__ __launch_bounds__(64) void finish_run_kernel(DevScalars* s, int which, StepRule rule) {
+  const unsigned long long m = fold_cdt(s + which);
+  StepState q = s[which];
+  if (q.pending && !q.halt) end_step(q, m, rule, 1, 0.0);
+  __syncthreads();                     // every lane has read before any writes
+  if (threadIdx.x == 0) {
+    static_cast<StepState&>(s[0]) = q;
+    s[1].err = 0;
+  }
+  const int k = threadIdx.x;
+  s[k / RED_SLOTS].cdt_red[red_index(k % RED_SLOTS)] = 0ull;
 }
 
 // Plain streaming copy, used to calibrate the HBM byte counters and to
@@ -142,7 +93,7 @@ struct pmx_hydro {
   double* dx;       // [nx | ny | nz]
   double* dtdx;
   double* inv_dl;
-  DevScalars* s;
+  DevScalars* s;    // the time state, and the other one of a 2-D run
   double* dt_in;    // device slots of an explicit step: dt, and Dts->invDt_hyp on entry
   hipStream_t stream;
   hipGraphExec_t graph;
@@ -280,8 +231,14 @@ void dispatch_rec(pmx_hydro* h, const StageArgs& a, int nblocks, int mode) {
   }
 }
 
+StepRule step_rule(const pmx_hydro* h) {
+  return {h->d.dims, h->d.cfl, h->d.cfl_max_var, h->d.first_dt};
+}
+
+// cur: the step's time state; prev: the previous step's (2-D main-loop
+// stages 1 and 2), or null.
 int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int mode, double w0,
-          double wc, int write_u, bool loop) {
+          double wc, int write_u, bool loop, DevScalars* cur, DevScalars* prev) {
   StageArgs a;
   a.Vin = Vin;
   a.V0 = V0;
@@ -309,9 +266,15 @@ int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int m
     a.tiles_z = p.n ? p.n : (h->nz + p.cz - 1) / p.cz;
   }
   a.write_u = write_u;
-  a.cdt_bits = h->s->cdt_red;
-  a.err = &h->s->err;
-  a.halt = loop ? &h->s->halt : nullptr;
+  a.cdt_bits = cur->cdt_red;
+  a.err = &cur->err;
+  // (stage 1 of a 2-D main-loop step sets cur->halt itself)
+  a.halt = loop && !(prev && mode == MODE_FIRST) ? &cur->halt : nullptr;
+  a.dx[0] = h->dx;
+  a.dx[1] = h->dx + h->nx;
+  a.cur = cur;
+  a.prev = prev;
+  a.rule = step_rule(h);
   // with the z schedule, 8 ceil(tiles / 8) workgroups per chunk (a whole
   // number per XCD; see stage_kernel)
   int nblocks = a.nzc ? 8 * ((a.tiles_x * a.tiles_y + 7) / 8) * a.nzc
@@ -340,10 +303,22 @@ int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int m
   return 0;
 }
 
-// One AdvanceStep: Src/Time_Stepping/rk_step.c:117-330.  V[0] holds V^n on
-// entry and V^{n+1} on exit.  In the main loop the previous step's
-// finish_kernel has prepared this one (dt/dx, cleared slots) unless the
-// run is just starting (with_prep).
+// The RK stages of one AdvanceStep: Src/Time_Stepping/rk_step.c:117-330.
+// V[0] holds V^n on entry and V^{n+1} on exit.
+int stages(pmx_hydro* h, bool loop, DevScalars* cur, DevScalars* prev) {
+  if (h->d.rk == 3) {
+    if (stage(h, h->V[0], h->V[0], h->V[1], MODE_FIRST, 0, 0, 1, loop, cur, prev)) return -1;
+    if (stage(h, h->V[1], h->V[0], h->V[2], MODE_WEIGHTED, 0.75, 0.25, 1, loop, cur, prev))
+      return -1;
+    return stage(h, h->V[2], h->V[0], h->V[0], MODE_THIRD, 0, 0, 1, loop, cur, nullptr);
+  }
+  if (stage(h, h->V[0], h->V[0], h->V[1], MODE_FIRST, 0, 0, 1, loop, cur, prev)) return -1;
+  return stage(h, h->V[1], h->V[0], h->V[0], MODE_WEIGHTED, 0.5, 0.5, 1, loop, cur, prev);
+}
+
+// One step through the dt/dx table.  In the main loop (dt_override null)
+// the previous step's finish_kernel has prepared this one (dt/dx, cleared
+// slots) unless the run is just starting (with_prep).
 int advance(pmx_hydro* h, const double* dt_override, bool with_prep) {
   int ntot = h->nx + h->ny + h->nz;
   const bool loop = dt_override == nullptr;
@@ -352,17 +327,33 @@ int advance(pmx_hydro* h, const double* dt_override, bool with_prep) {
                        h->dx, h->dtdx, ntot, dt_override);
     PMX_HIP_CHECK(hipGetLastError());
   }
-  if (h->d.rk == 3) {
-    if (stage(h, h->V[0], h->V[0], h->V[1], MODE_FIRST, 0, 0, 1, loop)) return -1;
-    if (stage(h, h->V[1], h->V[0], h->V[2], MODE_WEIGHTED, 0.75, 0.25, 1, loop)) return -1;
-    if (stage(h, h->V[2], h->V[0], h->V[0], MODE_THIRD, 0, 0, 1, loop)) return -1;
-  } else {
-    if (stage(h, h->V[0], h->V[0], h->V[1], MODE_FIRST, 0, 0, 1, loop)) return -1;
-    if (stage(h, h->V[1], h->V[0], h->V[0], MODE_WEIGHTED, 0.5, 0.5, 1, loop)) return -1;
+  if (stages(h, loop, h->s, nullptr)) return -1;
+  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(256), 0, h->stream, h->s, step_rule(h),
+                     loop ? 1 : 0, loop ? nullptr : dt_override + 1, h->dx, h->dtdx, ntot);
+  PMX_HIP_CHECK(hipGetLastError());
+  return 0;
+}
+
+// Steps first .. first + n - 1 of a main-loop run.  A 2-D step is its stage
+// kernels alone: the time state alternates between s[0] and s[1], each
+// step's stage 1 ending the one before (KH 64^2: 6.4 -> 4.2 us per step,
+// whose launches take about 2 us each).
+int run_steps(pmx_hydro* h, int first, int n) {
+  for (int q = first; q < first + n; q++) {
+    if (h->d.dims == 2) {
+      if (stages(h, true, h->s + (q + 1) % 2, h->s + q % 2)) return -1;
+    } else if (advance(h, nullptr, q == 0)) {
+      return -1;
+    }
   }
-  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(256), 0, h->stream, h->s, h->d.dims,
-                     h->d.cfl, h->d.cfl_max_var, h->d.first_dt, loop ? 1 : 0,
-                     loop ? nullptr : dt_override + 1, h->dx, h->dtdx, ntot);
+  return 0;
+}
+
+// After nsteps main-loop steps: the 2-D run's time state back in s[0].
+int end_run(pmx_hydro* h, int nsteps) {
+  if (h->d.dims != 2 || nsteps == 0) return 0;
+  hipLaunchKernelGGL(finish_run_kernel, dim3(1), dim3(64), 0, h->stream, h->s, nsteps % 2,
+                     step_rule(h));
   PMX_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -470,17 +461,16 @@ int pmx_hydro_create(const pmx_hydro_desc* desc, pmx_hydro** out) {
   CK(hipMalloc(&h->dx, sizeof(double) * ntot));
   CK(hipMalloc(&h->dtdx, sizeof(double) * ntot));
   CK(hipMalloc(&h->inv_dl, sizeof(double) * ntot));
-  CK(hipMalloc(&h->s, sizeof(DevScalars)));
+  CK(hipMalloc(&h->s, 2 * sizeof(DevScalars)));
   CK(hipMalloc(&h->dt_in, 2 * sizeof(double)));
   {
     std::vector<double> dx, inv;
     host_tables(desc, h->nx, h->ny, h->nz, dx, inv);
     CK(hipMemcpy(h->dx, dx.data(), sizeof(double) * ntot, hipMemcpyHostToDevice));
     CK(hipMemcpy(h->inv_dl, inv.data(), sizeof(double) * ntot, hipMemcpyHostToDevice));
-    DevScalars s0;
-    memset(&s0, 0, sizeof(s0));
-    s0.tstop = HUGE_VAL;
-    CK(hipMemcpy(h->s, &s0, sizeof(s0), hipMemcpyHostToDevice));
+    DevScalars s0[2] = {};
+    s0[0].tstop = HUGE_VAL;
+    CK(hipMemcpy(h->s, s0, sizeof(s0), hipMemcpyHostToDevice));
   }
   for (int q = 0; q < 3; q++) CK(hipMemset(h->V[q], 0, vbytes));
   CK(hipMemset(h->U, 0, vbytes));
@@ -635,12 +625,11 @@ int pmx_hydro_advance_step(pmx_hydro* h, double dt, double* inv_dt_hyp) {
 
 int pmx_hydro_run(pmx_hydro* h, int nsteps) {
   if (!h || nsteps < 0) { set_error("bad argument"); return -1; }
-  for (int n = 0; n < nsteps; n++)
-    if (advance(h, nullptr, n == 0)) return -1;
-  return 0;
+  return run_steps(h, 0, nsteps) || end_run(h, nsteps) ? -1 : 0;
 }
 
-// Steps per captured graph: a graph launch costs more than the few kernel
+// Steps per captured graph (an even number, so that a 2-D graph ends where
+// it began, in s[0]): a graph launch costs more than the few kernel
 // launches of one step saves (KH 256^2: 33 us per step replaying one step
 // per graph against 26 us eager), so a graph holds several steps.  Steps
 // after the run halts are no-ops on the device, as in the eager loop.
@@ -652,8 +641,7 @@ int pmx_hydro_run_graph(pmx_hydro* h, int nsteps) {
   if (nsteps >= GRAPH_STEPS && !h->have_graph) {
     hipGraph_t g;
     PMX_HIP_CHECK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    int rc = 0;
-    for (int q = 0; q < GRAPH_STEPS && !rc; q++) rc = advance(h, nullptr, q == 0);
+    const int rc = run_steps(h, 0, GRAPH_STEPS);
     hipError_t e = hipStreamEndCapture(h->stream, &g);
     if (rc) return -1;
     if (e != hipSuccess) { set_error(std::string("capture: ") + hipGetErrorString(e)); return -1; }
@@ -664,9 +652,11 @@ int pmx_hydro_run_graph(pmx_hydro* h, int nsteps) {
   int n = 0;
   for (; nsteps - n >= GRAPH_STEPS; n += GRAPH_STEPS)
     PMX_HIP_CHECK(hipGraphLaunch(h->graph, h->stream));
-  for (const int n0 = n; n < nsteps; n++)
-    if (advance(h, nullptr, n == n0)) return -1;
-  return 0;
+  if (n < nsteps) {
+    // (a 3-D remainder starts with its own prep launch, as step 0 does)
+    if (run_steps(h, 0, nsteps - n)) return -1;
+  }
+  return end_run(h, nsteps);
 }
 
 int pmx_hydro_sync(pmx_hydro* h) {
@@ -772,7 +762,7 @@ int pmx_hydro_advance_step_noalloc(const pmx_hydro_desc* desc, double* V, double
   std::vector<double> dx, inv;
   host_tables(desc, nx, ny, nz, dx, inv);
   DevScalars s0;
-  memset(&s0, 0, sizeof(s0));       // what the last call left is cleared
+  s0 = DevScalars{};                // what the last call left is cleared
   s0.tstop = HUGE_VAL;
   const double in[2] = {dt, inv_dt_hyp ? *inv_dt_hyp : 0.0};
   PMX_HIP_CHECK(hipMemcpyAsync(h.dx, dx.data(), sizeof(double) * ntot, hipMemcpyHostToDevice, 0));

@@ -23,6 +23,7 @@
 //
 // Layout in HBM: V, U are SoA [nv][nz][ny][nx] float64, interior only.
 #pragma once
+#include "../../include/plutomx.h"
 #include "pmx_common.h"
 #include "pmx_hd_math.h"
 
@@ -72,6 +73,86 @@ template <int DIMS>
 constexpr int tile_y() { return DIMS == 3 ? TILE_Y : PMX_TILE_Y_2D; }
 constexpr int NTHREADS = 256;
 
+// The time state of a grid, and the step reductions behind it.
+struct StepState {
+  double t;                      // g_time
+  double dt;                     // g_dt of the step being taken
+  double inv_dt_hyp;             // Dts->invDt_hyp of the last step
+  double tstop;                  // runtime.tstop
+  double dt_uncut;               // the dt a cut to tstop replaced
+  int err;                       // cons->prim flags of the step under way
+  int step_err;                  // cons->prim flags of the last completed step
+  int halt;                      // PMX_FLAG_DT_TOO_SMALL / PMX_FLAG_TSTOP once set (sticky):
+                                 // later main-loop steps are no-ops
+  int last;                      // the next step is the last one (dt clamped to tstop - t)
+  int pending;                   // a step has been taken and end_step not yet applied
+};
+struct DevScalars : StepState {
+  unsigned long long cdt_red[RED_SLOTS * RED_STRIDE];   // stage-1 C_dt maxima, spread
+                                                        // (words red_index(k), 0 = none)
+};
+
+// Src/main.c:226-229: the step that would reach tstop (to 1e-8 relative)
+// is the last one, and its dt is cut to land on tstop.
+__host__ __device__ inline void clamp_last_step(StepState& s) {
+  if ((s.t + s.dt) >= s.tstop * (1.0 - 1.e-8)) {
+    s.dt_uncut = s.dt;
+    s.dt = (s.tstop - s.t);
+    s.last = 1;
+  }
+}
+
+// NextTimeStep's parameters (pmx_hydro_desc)
+struct StepRule {
+  int ndim;
+  double cfl, cfl_max_var, first_dt;
+};
+
+// Src/update_stage.c:389-394 then Src/main.c:596-697 (NextTimeStep, no
+// parabolic terms, no cooling) and the time update of main.c:296, from the
+// step's C_dt maximum (bit pattern) and the Dts->invDt_hyp it folds into.
+// In the main loop (loop != 0) NextTimeStep's "dt is too small" quit
+// (main.c:672-683) halts the run, and so does the end of the step that
+// reached tstop; otherwise the next step's dt is cut to land on tstop when
+// it would pass it (main.c:226-229).
+__device__ __forceinline__ void end_step(StepState& s, unsigned long long cdt_bits,
+                                         const StepRule& r, int loop, double inv_in) {
+  double inv = dmax(inv_in, __longlong_as_double((long long)cdt_bits));
+  inv /= (double)r.ndim;
+  s.inv_dt_hyp = inv;
+  s.step_err = s.err;
+  s.err = 0;
+  s.pending = 0;
+  double dt = s.dt;
+  s.t += dt;
+  double dt_hyp = 1.0 / inv;
+  dt_hyp *= r.cfl;
+  double dtnext = dt_hyp;
+  dtnext = dmin(dtnext, r.cfl_max_var * dt);
+  if (r.cfl_max_var != 1.0) s.dt = dtnext;
+  if (!loop) return;
+  if (dtnext < r.first_dt * 1.e-9) s.halt |= PMX_FLAG_DT_TOO_SMALL;   // main.c:672-683
+  if (s.last) {
+    s.halt |= PMX_FLAG_TSTOP;
+    s.last = 0;
+  } else {
+    clamp_last_step(s);
+  }
+}
+
+// The C_dt maximum of a step, in every lane (each loads one slot; the
+// non-negative doubles order like their bit patterns).
+__device__ __forceinline__ unsigned long long fold_cdt(const DevScalars* s) {
+  static_assert(RED_SLOTS == 32, "one slot per lane of a half wavefront");
+  unsigned long long m = s->cdt_red[red_index(threadIdx.x & (RED_SLOTS - 1))];
+#pragma unroll
+  for (int off = RED_SLOTS / 2; off > 0; off >>= 1) {
+    const unsigned long long u = __shfl_xor(m, off);
+    m = u > m ? u : m;
+  }
+  return m;
+}
+
 struct StageArgs {
   const double* Vin;   // stage input, halo source
   const double* V0;    // V at the start of the step (U0 = P2C(V0)); may alias Vout
@@ -98,6 +179,14 @@ struct StageArgs {
   int* err;                      // OR of cons->prim floor flags
   const int* halt;               // main-loop steps: skip the stage once nonzero; null for a
                                  // step the caller drives (explicit dt)
+  // 2-D: every stage takes dt from `cur` and dx, so a step needs no dt/dx
+  // table and no launch of its own between two steps.  In the main loop
+  // stage 1 applies end_step to the previous step's state `prev` and writes
+  // the result to `cur`; stage 2 clears prev's reductions for the step
+  // after the next, which takes prev as its cur.
+  const double* dx[2];
+  DevScalars *cur, *prev;        // prev: main-loop stages 1 and 2, else null
+  StepRule rule;
 };
 
 template <int REC> struct RecTraits {
@@ -207,6 +296,32 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
   if (a.halt && *a.halt) return;       // the run has stopped (uniform over the launch)
 
   const int tid = threadIdx.x;
+  // 2-D: this step's dt, formed here from the previous step's reductions in
+  // the main loop's stage 1 (the update is the first to use it, so that the
+  // loads pass behind the states and faces)
+  double dt2 = 0.0;
+  bool live = true;
+  if constexpr (DIMS == 2) {
+    if (MODE == MODE_FIRST && a.prev) {
+      StepState q = *a.prev;
+      const unsigned long long m = fold_cdt(a.prev);
+      if (q.pending && !q.halt) end_step(q, m, a.rule, 1, 0.0);
+      live = q.halt == 0;
+      dt2 = q.dt;
+      if (blockIdx.x == 0 && tid == 0) {
+        DevScalars* c = a.cur;         // (c->err and the slots collect this step's)
+        c->t = q.t; c->dt = q.dt; c->inv_dt_hyp = q.inv_dt_hyp; c->tstop = q.tstop;
+        c->dt_uncut = q.dt_uncut; c->step_err = q.step_err; c->halt = q.halt; c->last = q.last;
+        c->pending = live ? 1 : 0;
+      }
+    } else {
+      dt2 = a.cur->dt;
+      if (MODE != MODE_FIRST && a.prev && blockIdx.x == 0) {
+        if (tid < RED_SLOTS) a.prev->cdt_red[red_index(tid)] = 0ull;
+        if (tid == 0) a.prev->err = 0;
+      }
+    }
+  }
   const bool owner = tid < NC;         // thread owns tile cell (tx, ty)
   const int tx = tid % TX, ty = tid / TX;
   const int ntile = a.tiles_x * a.tiles_y;
@@ -457,7 +572,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         for (int nv = 0; nv < NV; nv++) vpz[nv] = vpn[nv];
       }
 
-      if (valid) {
+      if (valid && live) {
         if (MODE == MODE_FIRST) prim_to_cons(vc, u, gmm1);
         if (!PMX_PREFETCH_U && MODE != MODE_FIRST) {
 #pragma unroll
@@ -470,7 +585,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         // x
         {
           const double* Fm = &sFx[ty * (TX + 1) + tx];   // face i-1/2; i+1/2 is Fm[1]
-          double scrh = a.dtdx[0][i];
+          double scrh = DIMS == 2 ? dt2 / a.dx[0][i] : a.dtdx[0][i];
           double rhs[NV];
 #pragma unroll
           for (int nv = 0; nv < NV; nv++) rhs[nv] = -scrh * (Fm[nv * NFX + 1] - Fm[nv * NFX]);
@@ -483,7 +598,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         // y
         {
           const double* Fm = &sPlane[ty * TX + tx];       // face j-1/2; j+1/2 is Fm[TX]
-          double scrh = a.dtdx[1][j];
+          double scrh = DIMS == 2 ? dt2 / a.dx[1][j] : a.dtdx[1][j];
           double rhs[NV];
 #pragma unroll
           for (int nv = 0; nv < NV; nv++) rhs[nv] = -scrh * (Fm[nv * NFY + TX] - Fm[nv * NFY]);
@@ -548,7 +663,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
       double m = sRed[0];
       for (int q = 1; q < NT / 64; q++) m = dmax(m, sRed[q]);
       // non-negative doubles order like their bit patterns
-      atomicMax(a.cdt_bits + red_index(blockIdx.x), (unsigned long long)__double_as_longlong(m));
+      if (DIMS == 3 || live)
+        atomicMax(a.cdt_bits + red_index(blockIdx.x), (unsigned long long)__double_as_longlong(m));
     }
   }
   if (fail) atomicOr(a.err, fail);
