@@ -193,18 +193,26 @@ int boundary_kind(const pmx_hydro_desc& d) {
 template <int DIMS, int REC, int SOLVER, int MODE>
 void launch_stage(pmx_hydro* h, const StageArgs& a, int nblocks) {
   const dim3 g(nblocks), b(NTHREADS);
-  switch (boundary_kind(h->d)) {
-    case BCK_OUTFLOW:
-      hipLaunchKernelGGL((stage_kernel<DIMS, REC, SOLVER, MODE, BCK_OUTFLOW, TILE_X,
-                                       tile_y<DIMS>(), NTHREADS>), g, b, 0, h->stream, a);
-      break;
-    case BCK_PERIODIC:
-      hipLaunchKernelGGL((stage_kernel<DIMS, REC, SOLVER, MODE, BCK_PERIODIC, TILE_X,
-                                       tile_y<DIMS>(), NTHREADS>), g, b, 0, h->stream, a);
-      break;
-    default:   // mixed sides: compiled in pmx_hydro_any.hip
-      launch_stage_any(DIMS, REC, SOLVER, MODE, a, nblocks, h->stream);
+  const int bck = boundary_kind(h->d);
+  if (bck == BCK_ANY) {   // mixed sides: compiled in pmx_hydro_any.hip
+    launch_stage_any(DIMS, REC, SOLVER, MODE, a, nblocks, h->stream);
+    return;
   }
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, b, 0, h->stream, a); };
+  auto by_bck = [&](auto ty) {
+    constexpr int TY = decltype(ty)::value;
+    if (bck == BCK_OUTFLOW)
+      launch(stage_kernel<DIMS, REC, SOLVER, MODE, BCK_OUTFLOW, TILE_X, TY, NTHREADS>);
+    else
+      launch(stage_kernel<DIMS, REC, SOLVER, MODE, BCK_PERIODIC, TILE_X, TY, NTHREADS>);
+  };
+  if constexpr (DIMS == 2) {
+    if (a.tile_y == TILE_Y_2D) {
+      by_bck(std::integral_constant<int, TILE_Y_2D>());
+      return;
+    }
+  }
+  by_bck(std::integral_constant<int, TILE_Y>());
 }
 
 template <int DIMS, int REC, int SOLVER>
@@ -253,8 +261,8 @@ int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int m
   a.inv_dl[0] = h->inv_dl; a.inv_dl[1] = h->inv_dl + h->nx; a.inv_dl[2] = h->inv_dl + h->nx + h->ny;
   a.w0 = w0; a.wc = wc;
   a.tiles_x = (h->nx + TILE_X - 1) / TILE_X;
-  const int ty = h->d.dims == 3 ? tile_y<3>() : tile_y<2>();
-  a.tiles_y = (h->ny + ty - 1) / ty;
+  a.tile_y = tile_height(h->d.dims, h->nx, h->ny);
+  a.tiles_y = (h->ny + a.tile_y - 1) / a.tile_y;
   a.nzc = 0;
   a.cz = 1;
   a.tiles_z = 1;

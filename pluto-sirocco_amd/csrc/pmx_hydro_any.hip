@@ -14,8 +14,16 @@ namespace {
 
 template <int DIMS, int REC, int SOLVER, int MODE>
 void launch(const StageArgs& a, int nblocks, hipStream_t st) {
-  hipLaunchKernelGGL((stage_kernel<DIMS, REC, SOLVER, MODE, BCK_ANY, TILE_X, tile_y<DIMS>(), NTHREADS>),
-                     dim3(nblocks), dim3(NTHREADS), 0, st, a);
+  const dim3 g(nblocks), b(NTHREADS);
+  if constexpr (DIMS == 2) {
+    if (a.tile_y == TILE_Y_2D) {
+      hipLaunchKernelGGL((stage_kernel<DIMS, REC, SOLVER, MODE, BCK_ANY, TILE_X, TILE_Y_2D,
+                                       NTHREADS>), g, b, 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((stage_kernel<DIMS, REC, SOLVER, MODE, BCK_ANY, TILE_X, TILE_Y, NTHREADS>), g,
+                     b, 0, st, a);
 }
 
 template <int DIMS, int REC, int SOLVER>

@@ -63,14 +63,19 @@ enum { MODE_FIRST = 0, MODE_WEIGHTED = 1, MODE_THIRD = 2 };
 #endif
 constexpr int TILE_X = PMX_TILE_X;
 constexpr int TILE_Y = PMX_TILE_Y;
-// 2-D grids take shorter tiles: KH 256^2 makes 512 tiles of 16 x 8, two
-// workgroups on every CU, where 16 x 14 made 304, two on 48 CUs and one on
-// the rest (21.6-22.6 vs 22.9-23.8 us per step, bit-identical)
+// 2-D grids too small to give every CU a 16 x 14 tile take shorter ones:
+// more workgroups, but only half of their threads own a cell.  us per step
+// of the short / tall tiles: KH 128^2 (80 tall tiles) 13.6 / 14.5 alone, 5.1
+// / 5.7 next to two other runs; 256^2 (304) 18.1 / 19.4 and 12.2 / 8.8;
+// 300 x 400 31 / 29 and 22 / 15; 512^2 56 / 43; 1024^2 197 / 136.
 #ifndef PMX_TILE_Y_2D
 #define PMX_TILE_Y_2D 8
 #endif
-template <int DIMS>
-constexpr int tile_y() { return DIMS == 3 ? TILE_Y : PMX_TILE_Y_2D; }
+constexpr int TILE_Y_2D = PMX_TILE_Y_2D;
+inline int tile_height(int dims, int nx, int ny) {
+  const int tall = ((nx + TILE_X - 1) / TILE_X) * ((ny + TILE_Y - 1) / TILE_Y);
+  return dims == 3 || tall >= 256 ? TILE_Y : TILE_Y_2D;
+}
 constexpr int NTHREADS = 256;
 
 // The time state of a grid, and the step reductions behind it.
@@ -166,6 +171,7 @@ struct StageArgs {
   const double* inv_dl[3];  // 1/dx per cell and direction
   double w0, wc;            // RK weights for MODE_WEIGHTED
   int cz;                   // z planes per workgroup (uniform chunks, nzc == 0)
+  int tile_y;               // tile height: TILE_Y, or TILE_Y_2D
   int tiles_x, tiles_y, tiles_z;
   // z chunks of unequal length (3-D, nzc > 0): chunk c is planes
   // [zc0[c], zc0[c+1]); each XCD's workgroups take its tiles chunk by

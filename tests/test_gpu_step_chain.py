@@ -59,3 +59,22 @@ def test_halted_run_goes_on_after_a_later_tstop():
         g.run(33, graph=True)
         assert h.get_time() == g.get_time() and h.get_time()[0] == 0.03
         assert np.array_equal(h.get_prim(), g.get_prim())
+
+
+@pytest.mark.parametrize("nx,recon,bc", [
+    ((256, 223, 1), setups.PLM, setups.BC_PERIODIC),      # 16 x 16 tall tiles: the rule's edge
+    ((240, 238, 1), setups.PLM, setups.BC_PERIODIC),      # 15 x 17 = 255: short ones
+    ((259, 230, 1), setups.PPM, setups.BC_OUTFLOW),       # ragged tall tiles
+    ((258, 227, 1), setups.PPM, setups.BC_REFLECTIVE),
+    ((700, 97, 1), setups.PLM, setups.BC_OUTFLOW)])
+def test_both_tile_heights(nx, recon, bc):
+    import plutomx
+    cfg = setups.HydroConfig(dims=2, nx=nx, recon=recon, limiter=setups.LIM_MC, rk=3,
+                             bc=(bc,) * 6, first_dt=1e-3)
+    V0 = setups.kelvin_helmholtz(cfg, seed=3)
+    with plutomx.Hydro(cfg) as h:
+        h.set_prim(V0)
+        h.set_time(0.0, cfg.first_dt)
+        h.run(3)
+        ref = refrun.run_oracle(cfg, V0, 3)
+        assert np.array_equal(h.get_prim(), ref["V"]) and h.get_time()[1] == ref["dt"]
