@@ -311,6 +311,7 @@ int stage(pmx_hydro* h, const double* Vin, const double* V0, double* Vout, int m
   for (int q = 0; q < 6; q++) a.bc[q] = h->d.bc[q];
   a.gamma = h->d.gamma;
   a.gmm1 = h->d.gamma - 1.0;
+  a.rg = recip2(a.gmm1, 1.0 / a.gmm1);
   a.dtdx[0] = h->dtdx; a.dtdx[1] = h->dtdx + h->nx; a.dtdx[2] = h->dtdx + h->nx + h->ny;
   a.inv_dl[0] = h->inv_dl; a.inv_dl[1] = h->inv_dl + h->nx; a.inv_dl[2] = h->inv_dl + h->nx + h->ny;
   a.w0 = w0; a.wc = wc;

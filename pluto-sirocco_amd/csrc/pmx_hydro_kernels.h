@@ -167,6 +167,7 @@ struct StageArgs {
   long long sv;        // stride between variables = nx*ny*nz
   int bc[6];
   double gamma, gmm1;
+  Recip2 rg;           // of gmm1
   const double* dtdx[3];    // dt/dx per cell and direction (this step)
   const double* inv_dl[3];  // 1/dx per cell and direction
   double w0, wc;            // RK weights for MODE_WEIGHTED
@@ -368,6 +369,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
     k1 = __builtin_amdgcn_readfirstlane(k1);
   }
   const double gamma = a.gamma, gmm1 = a.gmm1;
+  const Recip2 rg = a.rg;
 
   double cdt_max = 0.0;
   int fail = 0;
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         ppm_limit(p[2][nv], Ib, Ia, vpm[nv], vmm);                       // cell k0-1
         ppm_limit(p[3][nv], Iz[nv], Ib, vpz[nv], vm0[nv]);               // cell k0
       }
-      riemann<SOLVER, 2, DIMS>(vpm, vm0, gamma, gmm1, Fz, Fz[5], Fz[6]);
+      riemann<SOLVER, 2, DIMS>(vpm, vm0, gamma, rg, Fz, Fz[5], Fz[6]);
 #pragma unroll
       for (int s = 0; s < 3; s++)
 #pragma unroll
@@ -408,7 +410,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
       double vpm[NV], vmm[NV], vm0[NV];
       plm_states<REC>(p[0], p[1], p[2], vpm, vmm);   // cell k0-1
       plm_states<REC>(p[1], p[2], p[3], vpz, vm0);   // cell k0
-      riemann<SOLVER, 2, DIMS>(vpm, vm0, gamma, gmm1, Fz, Fz[5], Fz[6]);
+      riemann<SOLVER, 2, DIMS>(vpm, vm0, gamma, rg, Fz, Fz[5], Fz[6]);
 #pragma unroll
       for (int s = 0; s < 2; s++)
 #pragma unroll
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         vL[nv] = sStX[nv * NST + sl];
         vR[nv] = sStX[(5 + nv) * NST + sr];
       }
-      riemann<SOLVER, 0, DIMS>(vL, vR, gamma, gmm1, F, F[5], F[6]);
+      riemann<SOLVER, 0, DIMS>(vL, vR, gamma, rg, F, F[5], F[6]);
 #pragma unroll
       for (int q = 0; q < 7; q++) sFx[q * NFX + f] = F[q];
     };
@@ -529,7 +531,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         vL[nv] = sStY[nv * NST + sl];
         vR[nv] = sStY[(5 + nv) * NST + sr];
       }
-      riemann<SOLVER, 1, DIMS>(vL, vR, gamma, gmm1, F, F[5], F[6]);
+      riemann<SOLVER, 1, DIMS>(vL, vR, gamma, rg, F, F[5], F[6]);
 #pragma unroll
       for (int q = 0; q < 7; q++) sPlane[q * NFY + f] = F[q];
     };
@@ -573,7 +575,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(PMX_WAVES_PE
         } else {
           plm_states<REC>(w[0], w[1], w[2], vpn, vmn);                     // cell k+1
         }
-        riemann<SOLVER, 2, DIMS>(vpz, vmn, gamma, gmm1, Fzn, Fzn[5], Fzn[6]);
+        riemann<SOLVER, 2, DIMS>(vpz, vmn, gamma, rg, Fzn, Fzn[5], Fzn[6]);
 #pragma unroll
         for (int nv = 0; nv < NV; nv++) vpz[nv] = vpn[nv];
       }

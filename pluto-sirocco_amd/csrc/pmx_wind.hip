@@ -504,23 +504,6 @@ struct LfCell {
   double num1, num2;
 };
 
-// x / c for a c that many quotients share: r + l = 1 / c to twice the
-// precision, so that the first quotient is within an ulp and one correction
-// rounds it (Markstein).  The sign of a zero is that of the dividend's only
-// when it is positive, which the sums these quotients go into do not see.
-struct Recip2 {
-  double c, r, l;
-};
-
-__device__ __forceinline__ Recip2 recip2(double c, double r) {   // r = 1 / c, rounded
-  return {c, r, fma(-c, r, 1.0) * r};
-}
-
-__device__ __forceinline__ double div2(double x, const Recip2& k) {
-  const double q = fma(x, k.r, x * k.l);
-  return fma(fma(-q, k.c, x), k.r, q);
-}
-
 constexpr double LF_HI = 0x1p400;    // range of dvds: 0, or 2^-400 .. 2^400
 constexpr int LF_NMAX = 400;
 constexpr double LF_NUM_LO = 0x1p-100, LF_NUM_HI = 0x1p100;
