@@ -6,7 +6,9 @@
 //                         ghost storage), VGradCalc, PLM, HLLC + tracer,
 //                         spherical RHS, geometric / gravity / line-force
 //                         sources, RK combination, cons->prim and the
-//                         stage-1 CFL reduction.  One thread per cell.
+//                         stage-1 CFL reduction.  A workgroup per tile, its
+//                         edge states and fluxes shared through LDS.
+//   wind_lforce_*         the stage's line force, before it.
 //   wind_cool_kernel<M>   SplitSource cooling (BLONDIN or the plain
 //                         integrator) and the dt_cool reduction.
 //   wind_end_kernel       time update and NextTimeStep (every second step
@@ -27,17 +29,19 @@ namespace pmx {
 namespace wind {
 
 constexpr int NG = 2;          // ghost cells of the reference grid (PLM)
-constexpr int BX = 64, BY = 2; // stage-kernel workgroup
+constexpr int BX = 64, BY = 2; // workgroup of the kernels of one zone per thread
+// Stage-kernel tile.  Line force and stage of one RK stage, us, at 512 x 256
+// plain / production, 301 x 143 plain, 200 x 100 production: 32 x 8 76.6 /
+// 90.5, 47.3, 48.8; 16 x 16 77.6 / 91.2, 48.2, 48.5; 64 x 4 77.9 / 91.0,
+// 47.3, 53.7; 32 x 4 80.2 / 91.9, 49.2, 50.9.
+constexpr int SX = 32, SY = 8;
 constexpr int NLF = 5;         // line-force tables per (angle, cell)
 constexpr int FM_POINTS_MAX = 4096;   // fit points of a tabulated force multiplier
 
 // Waves per SIMD that the register allocation of the batch stage kernels
-// and the one-grid feature kernels targets.  The plain
-// stage kernel fits 2 waves by itself (200-226 VGPRs); kernels built with
-// characteristic limiting, the entropy switch, the tabulated multiplier or
-// Roe would take more than 256 registers and fall to 1 wave, so they are
-// capped and spill.  (With the line force still inside it, the batch
-// kernel took 276 registers and 1 wave; capped at 2 it ran 1.5x faster.)
+// targets: one of them (one row per tile, every feature) would take more
+// than 256 registers by itself and fall to 1 wave; it spills.  The one-grid
+// stage kernels take 156-240 registers, two waves, by themselves.
 #ifndef PMX_WIND_WAVES
 #define PMX_WIND_WAVES 2
 #endif
@@ -119,32 +123,57 @@ __device__ __forceinline__ void midplane_cell(const StageArgs& a, int im, double
 // sides, then x2 sides over the full x1 range, so corners see both):
 // reflective flips the normal velocity; WIND_INNER caps v_r at 0; WIND_POLE
 // reflects the velocities and takes rho and p from the first interior row.
+// In two steps, so that a thread can have the loads of several cells under
+// way: raw_issue loads, raw_state applies the rules.
+struct RawState {
+  double v[NVW], rho0, prs0;   // rho0, prs0: the column's first row (a WIND_POLE ghost cell)
+  int im, jm;
+  bool fr, ft;
+};
+
+__device__ __forceinline__ void raw_issue(const StageArgs& a, const double* __restrict__ V,
+                                          int jj, int ii, RawState& r) {
+  r.fr = r.ft = false;
+  r.im = map_bc_wind(ii, a.nr, a.bc[0], a.bc[1], r.fr);
+  r.jm = map_bc_wind(jj, a.nt, a.bc[2], a.bc[3], r.ft);
+  const double* p = V + (long long)r.jm * a.nr + r.im;
+#pragma unroll
+  for (int nv = 0; nv < NVW; nv++) r.v[nv] = p[nv * a.sv];
+  r.rho0 = r.prs0 = 0.0;
+  if (jj < 0 && a.bc[2] == BC_WIND_POLE) {
+    r.rho0 = V[RHO * a.sv + r.im];
+    r.prs0 = V[PRS * a.sv + r.im];
+  }
+}
+
 // Returns 1 when the floors changed an interior cell (used for the cell's
 // own Uc).
-__device__ __forceinline__ int ld6(const StageArgs& a, const double* __restrict__ V, int jj,
-                                   int ii, double* v) {
-  bool fr = false, ft = false;
-  int im = map_bc_wind(ii, a.nr, a.bc[0], a.bc[1], fr);
-  int jm = map_bc_wind(jj, a.nt, a.bc[2], a.bc[3], ft);
-  const double* p = V + (long long)jm * a.nr + im;
+__device__ __forceinline__ int raw_state(const StageArgs& a, int jj, int ii, const RawState& r,
+                                         double* v) {
 #pragma unroll
-  for (int nv = 0; nv < NVW; nv++) v[nv] = p[nv * a.sv];
+  for (int nv = 0; nv < NVW; nv++) v[nv] = r.v[nv];
   int changed = 0;
   if (a.k.dfloor > 0.0) changed = floor_cell(a.k, v);
-  if (a.k.midplane && jm == a.nt - 1) midplane_cell(a, im, v);
-  if (fr) v[VX1] = -v[VX1];
+  if (a.k.midplane && r.jm == a.nt - 1) midplane_cell(a, r.im, v);
+  if (r.fr) v[VX1] = -v[VX1];
   if (ii < 0 && a.bc[0] == BC_WIND_INNER) v[VX1] = dmin(v[VX1], 0.0);
-  if (ft) v[VX2] = -v[VX2];
+  if (r.ft) v[VX2] = -v[VX2];
   if (jj < 0 && a.bc[2] == BC_WIND_POLE) {
-    const double* q = V + im;          // row 0 of the same column
-    double w[NVW];
-#pragma unroll
-    for (int nv = 0; nv < NVW; nv++) w[nv] = q[nv * a.sv];
-    if (a.k.dfloor > 0.0) floor_cell(a.k, w);
+    double w[NVW] = {};
+    w[RHO] = r.rho0;
+    w[PRS] = r.prs0;
+    if (a.k.dfloor > 0.0) floor_cell(a.k, w);   // rho and p do not depend on the rest
     v[RHO] = w[RHO];
     v[PRS] = w[PRS];
   }
   return changed;
+}
+
+__device__ __forceinline__ int ld6(const StageArgs& a, const double* __restrict__ V, int jj,
+                                   int ii, double* v) {
+  RawState r;
+  raw_issue(a, V, jj, ii, r);
+  return raw_state(a, jj, ii, r, v);
 }
 
 __device__ __forceinline__ void ld6(const StageArgs& a, int jj, int ii, double* v) {
@@ -623,60 +652,233 @@ __device__ __forceinline__ void lforce_bins(const StageArgs& a, const LfCell& z,
   }
 }
 
-template <int STAGE, int FEAT>
-__device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, double& cdt,
+// A zone's two edge states in a DIR sweep (coefficients c), with its
+// entropy's behind them when the kernel carries it: l, v, r hold the zone
+// and its neighbours.
+template <int DIR, int FEAT>
+__device__ __forceinline__ void edge_states(const StageArgs& a, int j, int i, bool ent,
+                                            const double* l, const double* v, const double* r,
+                                            const double* c, double* vp, double* vm) {
+  plm_zone<DIR, FEAT & FEAT_CHAR>(a, j, i, l, v, r, c, vp, vm);
+  if ((FEAT & FEAT_ENT) && ent)        // scalars follow FLAG_MINMOD without characteristics
+    plm_scalar(l[NVW], v[NVW], r[NVW], c, !a.k.char_lim && minmod_zone(a, j, i), vp[NVW],
+               vm[NVW]);
+}
+
+// The interface between two zones: its flux, pressure and signal speed, then
+// the entropy flux (adv_flux.c:131-134).
+template <int DIR, int FEAT>
+__device__ __forceinline__ void edge_flux(const Const& k, bool ent, const double* vL,
+                                          const double* vR, bool hll, double* F) {
+  face<DIR, (FEAT & FEAT_ROE) != 0>(vL, vR, k, F, F[NVW], F[NVW + 1], hll);
+  if ((FEAT & FEAT_ENT) && ent)
+    F[NVW + 2] = F[RHO] >= 0.0 ? vL[NVW] * F[RHO] : vR[NVW] * F[RHO];
+}
+
+// A tile of TX x TY zones at (i0, j0), one thread each.  The tile and the two
+// zones around it are brought into LDS once, all loads under way together; a
+// thread then reconstructs its own zone in both sweeps and solves its lower
+// interface of each, and the upper edge states of the zones below and the
+// fluxes of the interfaces above come through LDS.  The zones and interfaces
+// along the tile's rim are an extra pass of a few threads.
+//
+// What bounds it is waiting: 512 x 256 zones are two wavefronts per SIMD,
+// each with a chain of loads, barriers and dependent FP64 operations.  Per
+// stage launch at 512 x 256 (plain): 21.6 us with every thread forming its
+// four interfaces from nine zones, whose loads each waited for the boundary
+// rules of the one before (2.6 k vector instructions per wavefront); 19.5 us
+// with the interfaces shared (1.6 k); 16.9 us with the loads together.
+// Bringing the update's geometry in with them gained nothing.
+template <int STAGE, int FEAT, int TX, int TY>
+__device__ __forceinline__ void tile_stage(const StageArgs& a, int i0, int j0, double& cdt,
                                            int& flags) {
+  constexpr int NT = TX * TY, PW = TX + 4, PN = PW * (TY + 4);
+  constexpr int NS = NVW + ((FEAT & FEAT_ENT) ? 1 : 0), NF = NS + 2;
+  constexpr int RIM1 = 2 * TX + 64 <= NT ? NT - 64 : 0;  // first thread of the x1 rim
+  static_assert(NT >= TX && 2 * TY <= NT - RIM1, "the rim's zones find threads");
+  constexpr int BUF = NS * PN > 2 * NF * NT ? NS * PN : 2 * NF * NT;
+  __shared__ double sBuf[BUF];               // the states, then the upper interfaces
+  __shared__ double sP1[NS][(TX + 1) * TY], sP2[NS][TX * (TY + 1)];   // upper edge states
+  __shared__ unsigned char sFloored[STAGE == 2 ? PN : 1];
+  double* const sF1 = sBuf;
+  double* const sF2 = sBuf + NF * NT;
+  const Const& k = a.k;
+  const Tables& T = a.T;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TX + tx;
+  const int i = i0 + tx, j = j0 + ty, I = i + NG, J = j + NG;
+  const long long cell = (long long)j * a.nr + i;
+  const bool in = i < a.nr && j < a.nt;
+  // the zone behind the last one has the last interface
+  const bool in1 = i <= a.nr && j < a.nt, in2 = i < a.nr && j <= a.nt;
+  const bool ent = (FEAT & FEAT_ENT) && k.ent;
+
+  // ---- states ------------------------------------------------------------
+  constexpr int ROUNDS = (PN + NT - 1) / NT;
+  double g1r = 0.0, g2t = 0.0, Ui[STAGE == 2 ? NVW : 1], Vi[STAGE == 2 ? NVW : 1];
+  double c1[6], c2[6];
   {
-    const Const& k = a.k;
-    const Tables& T = a.T;
-    const double dt = a.s->dt;
-    const int I = i + NG, J = j + NG;
-    const long long cell = (long long)j * a.nr + i;
-
-    // ---- x1 stencil and reconstruction -------------------------------
-    double vc[NVW], w1[NVW], e1[NVW];
-    const int floored = ld6(a, a.Vin, j, i, vc);
-    ld6(a, j, i - 1, w1);
-    ld6(a, j, i + 1, e1);
-    const bool ent = (FEAT & FEAT_ENT) && k.ent;
-    const bool smm = !k.char_lim;      // scalars follow FLAG_MINMOD without characteristics
-    double sc = 0.0, sw1 = 0.0, se1 = 0.0;
-    if (ent) {
-      sc = entropy_of(vc, k.gamma);
-      sw1 = entropy_of(w1, k.gamma);
-      se1 = entropy_of(e1, k.gamma);
-    }
-    double c[6];
-    double vpi[NVW], vmi[NVW];
-    ldc(T.pr, a.nr, I, c);
-    plm_zone<0, FEAT & FEAT_CHAR>(a, j, i, w1, vc, e1, c, vpi, vmi);
-
-    // ---- the line force of both sweeps, from the line-force kernel
-    const double g1r = a.glf[cell], g2t = a.glf[a.sv + cell];
-
-    // ---- x1 faces i-1/2 and i+1/2 --------------------------------------
-    double rhs1[NVW], Fm[NVW], Fp[NVW], pm, pp, cm1, cp1;
-    double fem = 0.0, fep = 0.0;       // entropy fluxes (adv_flux.c:131-134)
-    {
-      double w2[NVW], e2[NVW], vpl[NVW], vml[NVW], vpr[NVW], vmr[NVW];
-      ld6(a, j, i - 2, w2);
-      ld6(a, j, i + 2, e2);
-      double cl[6], cr[6];
-      ldc(T.pr, a.nr, I - 1, cl);
-      plm_zone<0, FEAT & FEAT_CHAR>(a, j, i - 1, w2, w1, vc, cl, vpl, vml);
-      ldc(T.pr, a.nr, I + 1, cr);
-      plm_zone<0, FEAT & FEAT_CHAR>(a, j, i + 1, vc, e1, e2, cr, vpr, vmr);
-      face<0, (FEAT & FEAT_ROE) != 0>(vpl, vmi, k, Fm, pm, cm1, hll_interface(a, j, i - 1, j, i));
-      face<0, (FEAT & FEAT_ROE) != 0>(vpi, vmr, k, Fp, pp, cp1, hll_interface(a, j, i, j, i + 1));
-      if (ent) {
-        double spl, sml, spi, smi, spr, smr;
-        plm_scalar(entropy_of(w2, k.gamma), sw1, sc, cl, smm && minmod_zone(a, j, i - 1), spl, sml);
-        plm_scalar(sw1, sc, se1, c, smm && minmod_zone(a, j, i), spi, smi);
-        plm_scalar(sc, se1, entropy_of(e2, k.gamma), cr, smm && minmod_zone(a, j, i + 1), spr, smr);
-        fem = Fm[RHO] >= 0.0 ? spl * Fm[RHO] : smi * Fm[RHO];
-        fep = Fp[RHO] >= 0.0 ? spi * Fp[RHO] : smr * Fp[RHO];
+    RawState raw[ROUNDS];
+    auto zone = [&](int r, int& jz, int& iz) {       // whether the tile's zone is on the grid
+      const int z = tid + r * NT;
+      jz = j0 - NG + z / PW;
+      iz = i0 - NG + z % PW;
+      return z < PN && iz < a.nr + NG && jz < a.nt + NG;
+    };
+    int jz, iz;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+      if (zone(r, jz, iz)) raw_issue(a, a.Vin, jz, iz, raw[r]);
+    // what the update reads is loaded here too
+    if (in1) ldc(T.pr, a.nr, I, c1);
+    if (in2) ldc(T.pt, a.nt, J, c2);
+    if (in) {
+      g1r = a.glf[cell];               // the line force of both sweeps
+      g2t = a.glf[a.sv + cell];
+      if (STAGE == 2) {
+#pragma unroll
+        for (int nv = 0; nv < NVW; nv++) {
+          Ui[nv] = a.U[nv * a.sv + cell];
+          Vi[nv] = a.Vn[nv * a.sv + cell];
+        }
       }
     }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++)
+      if (zone(r, jz, iz)) {
+        double v[NVW];
+        const int z = tid + r * NT;
+        const int fl = raw_state(a, jz, iz, raw[r], v);
+        if (STAGE == 2) sFloored[z] = (unsigned char)fl;
+#pragma unroll
+        for (int nv = 0; nv < NVW; nv++) sBuf[nv * PN + z] = v[nv];
+        if ((FEAT & FEAT_ENT) && ent) sBuf[(NS - 1) * PN + z] = entropy_of(v, k.gamma);
+      }
+  }
+  __syncthreads();
+
+  // ---- reconstruction ----------------------------------------------------
+  auto state = [&](int z, double* v) {
+#pragma unroll
+    for (int q = 0; q < NS; q++) v[q] = sBuf[q * PN + z];
+  };
+  const int zc = (ty + NG) * PW + tx + NG;
+  double vc[NS], vsr = 0.0, vst = 0.0, vsp = 0.0;   // centre; x1 face averages (rho, v2, v3)
+  double vm1[NS], vm2[NS], xm1[NS], xm2[NS];        // lower edges of the own and rim zones
+  const int floored = STAGE == 2 && in ? sFloored[zc] : 0;
+  if (in1 || in2) state(zc, vc);
+  if (in1) {
+    double l[NS], r[NS], vp[NS];
+    state(zc - 1, l);
+    state(zc + 1, r);
+    edge_states<0, FEAT>(a, j, i, ent, l, vc, r, c1, vp, vm1);
+#pragma unroll
+    for (int q = 0; q < NS; q++) sP1[q][ty * (TX + 1) + tx + 1] = vp[q];
+    vsr = 0.5 * (vp[RHO] + vm1[RHO]);
+    vst = 0.5 * (vp[VX2] + vm1[VX2]);
+    vsp = 0.5 * (vp[VX3] + vm1[VX3]);
+  }
+  if (in2) {
+    double l[NS], r[NS], vp[NS];
+    state(zc - PW, l);
+    state(zc + PW, r);
+    edge_states<1, FEAT>(a, j, i, ent, l, vc, r, c2, vp, vm2);
+#pragma unroll
+    for (int q = 0; q < NS; q++) sP2[q][tid + TX] = vp[q];
+  }
+  for (int e = tid; e < 2 * TX; e += NT) {           // x2 rim: the row below, the row above
+    const int x = e < TX ? e : e - TX, y = e < TX ? -1 : TY, iz = i0 + x, jz = j0 + y;
+    if (iz < a.nr && jz <= a.nt) {
+      const int z = (y + NG) * PW + x + NG;
+      double l[NS], v[NS], r[NS], vp[NS], c[6];
+      ldc(T.pt, a.nt, jz + NG, c);
+      state(z - PW, l);
+      state(z, v);
+      state(z + PW, r);
+      edge_states<1, FEAT>(a, jz, iz, ent, l, v, r, c, vp, xm2);
+      if (e < TX) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) sP2[q][e] = vp[q];
+      }
+    }
+  }
+  const int e1 = tid - RIM1;                         // x1 rim: the column before, the one behind
+  if (e1 >= 0 && e1 < 2 * TY) {
+    const int y = e1 < TY ? e1 : e1 - TY, x = e1 < TY ? -1 : TX, iz = i0 + x, jz = j0 + y;
+    if (jz < a.nt && iz <= a.nr) {
+      const int z = (y + NG) * PW + x + NG;
+      double l[NS], v[NS], r[NS], vp[NS], c[6];
+      ldc(T.pr, a.nr, iz + NG, c);
+      state(z - 1, l);
+      state(z, v);
+      state(z + 1, r);
+      edge_states<0, FEAT>(a, jz, iz, ent, l, v, r, c, vp, xm1);
+      if (e1 < TY) {
+#pragma unroll
+        for (int q = 0; q < NS; q++) sP1[q][e1 * (TX + 1)] = vp[q];
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- interfaces --------------------------------------------------------
+  double Fm[NF], Gm[NF];
+  if (in1) {
+    double vL[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) vL[q] = sP1[q][ty * (TX + 1) + tx];
+    edge_flux<0, FEAT>(k, ent, vL, vm1, hll_interface(a, j, i - 1, j, i), Fm);
+    if (tx > 0) {
+#pragma unroll
+      for (int q = 0; q < NF; q++) sF1[q * NT + tid - 1] = Fm[q];
+    }
+  }
+  if (in2) {
+    double vL[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) vL[q] = sP2[q][tid];
+    edge_flux<1, FEAT>(k, ent, vL, vm2, hll_interface(a, j - 1, i, j, i), Gm);
+    if (ty > 0) {
+#pragma unroll
+      for (int q = 0; q < NF; q++) sF2[q * NT + tid - TX] = Gm[q];
+    }
+  }
+  for (int e = tid; e < 2 * TX; e += NT) {
+    const int iz = i0 + e - TX, jz = j0 + TY;
+    if (e >= TX && iz < a.nr && jz <= a.nt) {
+      double vL[NS], F[NF];
+#pragma unroll
+      for (int q = 0; q < NS; q++) vL[q] = sP2[q][e - TX + TY * TX];
+      edge_flux<1, FEAT>(k, ent, vL, xm2, hll_interface(a, jz - 1, iz, jz, iz), F);
+#pragma unroll
+      for (int q = 0; q < NF; q++) sF2[q * NT + e - TX + (TY - 1) * TX] = F[q];
+    }
+  }
+  if (e1 >= TY && e1 < 2 * TY) {
+    const int jz = j0 + e1 - TY, iz = i0 + TX;
+    if (jz < a.nt && iz <= a.nr) {
+      double vL[NS], F[NF];
+#pragma unroll
+      for (int q = 0; q < NS; q++) vL[q] = sP1[q][(e1 - TY) * (TX + 1) + TX];
+      edge_flux<0, FEAT>(k, ent, vL, xm1, hll_interface(a, jz, iz - 1, jz, iz), F);
+#pragma unroll
+      for (int q = 0; q < NF; q++) sF1[q * NT + (e1 - TY) * TX + TX - 1] = F[q];
+    }
+  }
+  __syncthreads();
+  if (!in) return;
+
+  {
+    const double dt = a.s->dt;
+    double Fp[NF], Gp[NF];
+#pragma unroll
+    for (int q = 0; q < NF; q++) { Fp[q] = sF1[q * NT + tid]; Gp[q] = sF2[q * NT + tid]; }
+    const double pm = Fm[NVW], pp = Fp[NVW], cm1 = Fm[NVW + 1], cp1 = Fp[NVW + 1];
+    const double qm = Gm[NVW], qp = Gp[NVW], cm2 = Gm[NVW + 1], cp2 = Gp[NVW + 1];
+    const double fem = ent ? Fm[NF - 1] : 0.0, fep = ent ? Fp[NF - 1] : 0.0;
+    const double gem = ent ? Gm[NF - 1] : 0.0, gep = ent ? Gp[NF - 1] : 0.0;
+
+    // ---- x1 sweep -------------------------------------------------------
+    double rhs1[NVW], rhs2[NVW];
     double rhs1e = 0.0;
     {
       const double dmu = T.dmu[J];
@@ -695,50 +897,19 @@ __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, dou
       rhs1[VX1] -= dtdl * (pp - pm);
       rhs1[VX3] /= fabs(T.x1[I]);
       // rhs_source.c:227-297
-      double vs[NVW];
-#pragma unroll
-      for (int nv = 0; nv < NVW; nv++) vs[nv] = 0.5 * (vpi[nv] + vmi[nv]);
       double r_1 = 1.0 / T.x1[I];
-      double vphi = vs[VX3];
-      double Sm = vs[RHO] * (vs[VX2] * vs[VX2] + vphi * vphi);
+      double vphi = vsp;
+      double Sm = vsr * (vst * vst + vphi * vphi);
       Sm += -0.0 - 0.0;
       rhs1[VX1] += dt * Sm * r_1;
       double g0 = -1.0 * k.gm_code / (T.x1[I] * T.x1[I]);
-      rhs1[VX1] += dt * vs[RHO] * g0;
+      rhs1[VX1] += dt * vsr * g0;
       rhs1[ENG] += dt * 0.5 * (Fp[RHO] + Fm[RHO]) * g0;
-      rhs1[VX1] += dt * vs[RHO] * g1r;
+      rhs1[VX1] += dt * vsr * g1r;
       rhs1[ENG] += dt * 0.5 * (Fp[RHO] + Fm[RHO]) * g1r;
     }
 
-    // ---- x2 faces j-1/2 and j+1/2 --------------------------------------
-    double rhs2[NVW], Gm[NVW], Gp[NVW], qm, qp, cm2, cp2;
-    double gem = 0.0, gep = 0.0;
-    {
-      double s1[NVW], n1[NVW], s2[NVW], n2[NVW];
-      ld6(a, j - 1, i, s1);
-      ld6(a, j + 1, i, n1);
-      ld6(a, j - 2, i, s2);
-      ld6(a, j + 2, i, n2);
-      double vpc[NVW], vmc[NVW], vpl[NVW], vml[NVW], vpr[NVW], vmr[NVW];
-      double cl[6], cr[6];
-      ldc(T.pt, a.nt, J, c);
-      plm_zone<1, FEAT & FEAT_CHAR>(a, j, i, s1, vc, n1, c, vpc, vmc);
-      ldc(T.pt, a.nt, J - 1, cl);
-      plm_zone<1, FEAT & FEAT_CHAR>(a, j - 1, i, s2, s1, vc, cl, vpl, vml);
-      ldc(T.pt, a.nt, J + 1, cr);
-      plm_zone<1, FEAT & FEAT_CHAR>(a, j + 1, i, vc, n1, n2, cr, vpr, vmr);
-      face<1, (FEAT & FEAT_ROE) != 0>(vpl, vmc, k, Gm, qm, cm2, hll_interface(a, j - 1, i, j, i));
-      face<1, (FEAT & FEAT_ROE) != 0>(vpc, vmr, k, Gp, qp, cp2, hll_interface(a, j, i, j + 1, i));
-      if (ent) {
-        const double ss1 = entropy_of(s1, k.gamma), sn1 = entropy_of(n1, k.gamma);
-        double spl, sml, spc, smc, spr, smr;
-        plm_scalar(entropy_of(s2, k.gamma), ss1, sc, cl, smm && minmod_zone(a, j - 1, i), spl, sml);
-        plm_scalar(ss1, sc, sn1, c, smm && minmod_zone(a, j, i), spc, smc);
-        plm_scalar(sc, sn1, entropy_of(n2, k.gamma), cr, smm && minmod_zone(a, j + 1, i), spr, smr);
-        gem = Gm[RHO] >= 0.0 ? spl * Gm[RHO] : smc * Gm[RHO];
-        gep = Gp[RHO] >= 0.0 ? spc * Gp[RHO] : smr * Gp[RHO];
-      }
-    }
+    // ---- x2 sweep -------------------------------------------------------
     double rhs2e = 0.0;
     {
       double base = fabs(T.x1[I]) * T.dx1[I];
@@ -790,7 +961,7 @@ __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, dou
       p2c6((STAGE == 2 && mid_row) ? vfl : vc, u, k.gmm1);
     } else {
 #pragma unroll
-      for (int nv = 0; nv < NVW; nv++) u[nv] = a.U[nv * a.sv + cell];
+      for (int nv = 0; nv < NVW; nv++) u[nv] = Ui[STAGE == 2 ? nv : 0];
     }
 #pragma unroll
     for (int nv = 0; nv < NVW; nv++) u[nv] += rhs1[nv];
@@ -799,7 +970,7 @@ __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, dou
     if (STAGE == 2) {
       double vn[NVW], u0[NVW];
 #pragma unroll
-      for (int nv = 0; nv < NVW; nv++) vn[nv] = a.Vn[nv * a.sv + cell];
+      for (int nv = 0; nv < NVW; nv++) vn[nv] = Vi[STAGE == 2 ? nv : 0];
       if (k.dfloor > 0.0) floor_cell(k, vn);   // U0 was formed after the floors
       if (mid_row) midplane_cell(a, i, vn);    // and the midplane row
       p2c6(vn, u0, k.gmm1);
@@ -812,7 +983,7 @@ __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, dou
       // stage-1 value, or for a zone the floors changed rho times the
       // entropy the stage-1 cons->prim left (Ue / rho of the stage-1 U)
       double ue;
-      if (STAGE == 1) ue = vc[RHO] * sc;
+      if (STAGE == 1) ue = vc[RHO] * vc[NS - 1];
       else if (floored) ue = (mid_row ? vfl[RHO] : vc[RHO]) *
                              (a.Ue[cell] * (1.0 / a.U[RHO * a.sv + cell]));
       else ue = a.Ue[cell];
@@ -821,7 +992,7 @@ __device__ __forceinline__ void cell_stage(const StageArgs& a, int i, int j, dou
       if (STAGE == 2) {
         double vn[NVW];
 #pragma unroll
-        for (int nv = 0; nv < NVW; nv++) vn[nv] = a.Vn[nv * a.sv + cell];
+        for (int nv = 0; nv < NVW; nv++) vn[nv] = Vi[STAGE == 2 ? nv : 0];
         if (k.dfloor > 0.0) floor_cell(k, vn);
         if (mid_row) midplane_cell(a, i, vn);
         const double u0e = vn[RHO] * entropy_of(vn, k.gamma);
@@ -913,12 +1084,10 @@ __global__ __launch_bounds__(BX* BY) void wind_flag_kernel(StageArgs a, unsigned
 template <int STAGE, int FEAT>
 __device__ __forceinline__ void stage_grid(const StageArgs& a) {
   if (a.loop && a.s->halt) return;     // the run has stopped (uniform over the launch)
-  const int i = blockIdx.x * BX + threadIdx.x;
-  const int j = blockIdx.y * BY + threadIdx.y;
   double cdt = 0.0;
   int flags = 0;
-  if (i < a.nr && j < a.nt) cell_stage<STAGE, FEAT>(a, i, j, cdt, flags);
-  if (block_reduce_stage<STAGE, BX * BY>(a.s, cdt, flags)) {
+  tile_stage<STAGE, FEAT, SX, SY>(a, blockIdx.x * SX, blockIdx.y * SY, cdt, flags);
+  if (block_reduce_stage<STAGE, SX * SY>(a.s, cdt, flags)) {
     if (STAGE == 2 && blockIdx.x == 0 && blockIdx.y == 0) {
       // update_stage.c:389-394: invDt = MAX(invDt, C_dt) over the domain,
       // then / DIMENSIONS (stage-1 values, complete when stage 2 runs)
@@ -930,19 +1099,8 @@ __device__ __forceinline__ void stage_grid(const StageArgs& a) {
   }
 }
 
-// The plain stage fits 2 waves per SIMD by itself (forcing the attribute
-// on it cost 13% while the line force was still part of it); with
-// characteristic limiting, the entropy switch or the
-// tabulated force multiplier the allocation grows past 256 registers
-// (VGPRs + AGPRs) and falls to 1 wave unless capped.
 template <int STAGE, int FEAT>
-__global__ __launch_bounds__(BX* BY) void wind_stage_kernel(StageArgs a) {
-  stage_grid<STAGE, FEAT>(a);
-}
-
-template <int STAGE, int FEAT>
-__global__ __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(PMX_WIND_WAVES, PMX_WIND_WAVES)))
-void wind_stage_kernel_w(StageArgs a) {
+__global__ __launch_bounds__(SX* SY) void wind_stage_kernel(StageArgs a) {
   stage_grid<STAGE, FEAT>(a);
 }
 
@@ -1358,20 +1516,6 @@ int features(const pmx_wind* w) {
          (w->k.fm_points > 0 ? FEAT_TAB : 0) | (w->k.roe ? FEAT_ROE : 0);
 }
 
-// Stage 1 of the feature kernels needs the 2-wave cap (it also carries the
-// CFL reduction), and so do the stage-2 kernels that would otherwise take
-// accumulation registers and drop to one wave per SIMD (characteristic
-// limiting with the entropy switch, and the tabulated force multiplier);
-// stage 2 of the others fits 2 waves by itself, where the cap only adds
-// spills.
-template <int STAGE, int FEAT>
-void launch_feat(pmx_wind* w, dim3 grid, dim3 block, const StageArgs& a) {
-  if (STAGE == 1 || (FEAT & FEAT_TAB) || (FEAT & 3) == 3)
-    hipLaunchKernelGGL((wind_stage_kernel_w<STAGE, FEAT>), grid, block, 0, w->stream, a);
-  else
-    hipLaunchKernelGGL((wind_stage_kernel<STAGE, FEAT>), grid, block, 0, w->stream, a);
-}
-
 // Four wavefronts share the bins of 64 zones while the zones alone make
 // fewer than one and a half wavefronts per SIMD (8 k cells: 15 against 30 us,
 // 43 k: 29 against 50, 74 k: 45 against 52, 98 k: 54 both ways, 131 k: 75
@@ -1404,18 +1548,22 @@ void launch_stage(pmx_wind* w, dim3 grid, dim3 block, const StageArgs& a) {
     default:
       hipLaunchKernelGGL((wind_lforce_kernel<FEAT_CHAR | FEAT_TAB>), grid, block, 0, w->stream, a);
   }
+  const dim3 sg((w->nr + SX - 1) / SX, (w->nt + SY - 1) / SY), sb(SX, SY);
+#define PMX_FEAT(F) \
+  hipLaunchKernelGGL((wind_stage_kernel<STAGE, F>), sg, sb, 0, w->stream, a)
   switch (features(w)) {
-    case 0: hipLaunchKernelGGL((wind_stage_kernel<STAGE, 0>), grid, block, 0, w->stream, a); break;
-    case 1: launch_feat<STAGE, 1>(w, grid, block, a); break;
-    case 2: launch_feat<STAGE, 2>(w, grid, block, a); break;
-    case 3: launch_feat<STAGE, 3>(w, grid, block, a); break;
-    case FEAT_ROE: launch_feat<STAGE, FEAT_ROE>(w, grid, block, a); break;
+    case 0: PMX_FEAT(0); break;
+    case 1: PMX_FEAT(1); break;
+    case 2: PMX_FEAT(2); break;
+    case 3: PMX_FEAT(3); break;
+    case FEAT_ROE: PMX_FEAT(FEAT_ROE); break;
     // the tabulated force multiplier, or Roe with other features: one
     // kernel with every feature (grids still check each)
     default:
-      if (features(w) & FEAT_ROE) launch_feat<STAGE, 15>(w, grid, block, a);
-      else launch_feat<STAGE, 7>(w, grid, block, a);
+      if (features(w) & FEAT_ROE) PMX_FEAT(15);
+      else PMX_FEAT(7);
   }
+#undef PMX_FEAT
 }
 
 int advance(pmx_wind* w, bool loop) {
@@ -2211,10 +2359,9 @@ void wind_batch_stage_kernel(const StageArgs* __restrict__ args, const int* __re
     const int tx_n = (a.nr + TBX - 1) / TBX;
     const int local = item - tile_off[g];
     const int ty = local / tx_n, tx = local - ty * tx_n;
-    const int i = tx * TBX + threadIdx.x, j = ty * TBY + threadIdx.y;
     double cdt = 0.0;
     int flags = 0;
-    if (i < a.nr && j < a.nt) cell_stage<STAGE, FEAT>(a, i, j, cdt, flags);
+    tile_stage<STAGE, FEAT, TBX, TBY>(a, tx * TBX, ty * TBY, cdt, flags);
     block_reduce_stage<STAGE, TBX * TBY>(a.s, cdt, flags);
   }
 }
