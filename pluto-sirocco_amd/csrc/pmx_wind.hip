@@ -180,17 +180,30 @@ __device__ __forceinline__ void ld6(const StageArgs& a, int jj, int ii, double* 
   ld6(a, a.Vin, jj, ii, v);
 }
 
-__device__ __forceinline__ void ld_vel(const StageArgs& a, int jj, int ii, double& v1,
-                                       double& v2) {
-  bool fr = false, ft = false;
-  int im = map_bc_wind(ii, a.nr, a.bc[0], a.bc[1], fr);
-  int jm = map_bc_wind(jj, a.nt, a.bc[2], a.bc[3], ft);
-  const double* p = a.Vin + (long long)jm * a.nr + im;
-  v1 = p[VX1 * a.sv];
-  v2 = p[VX2 * a.sv];
+// The velocities alone, in the same two steps.
+struct RawVel {
+  double rho, v1, v2;
+  int im, jm;
+  bool fr, ft;
+};
+
+__device__ __forceinline__ void vel_issue(const StageArgs& a, int jj, int ii, RawVel& r) {
+  r.fr = r.ft = false;
+  r.im = map_bc_wind(ii, a.nr, a.bc[0], a.bc[1], r.fr);
+  r.jm = map_bc_wind(jj, a.nt, a.bc[2], a.bc[3], r.ft);
+  const double* p = a.Vin + (long long)r.jm * a.nr + r.im;
+  r.v1 = p[VX1 * a.sv];
+  r.v2 = p[VX2 * a.sv];
+  r.rho = p[RHO * a.sv];
+}
+
+__device__ __forceinline__ void vel_state(const StageArgs& a, int ii, const RawVel& r,
+                                          double& v1, double& v2) {
+  v1 = r.v1;
+  v2 = r.v2;
   if (a.k.dfloor > 0.0) {
     // floor_cell's velocity scaling, which needs only rho
-    double rho = p[RHO * a.sv];
+    double rho = r.rho;
     if (rho < a.k.dfloor) {
       if (rho < 0.0) rho = a.k.dfloor;
       const double dfact = rho / a.k.dfloor;
@@ -198,14 +211,14 @@ __device__ __forceinline__ void ld_vel(const StageArgs& a, int jj, int ii, doubl
       v2 = dfact * v2;
       rho = a.k.dfloor;
     }
-    if (a.k.midplane && jm == a.nt - 1) {   // midplane_cell's velocities
-      v2 = (rho * v2) / a.T.mid[im];
+    if (a.k.midplane && r.jm == a.nt - 1) {   // midplane_cell's velocities
+      v2 = (rho * v2) / a.T.mid[r.im];
       v1 = 0.0;
     }
   }
-  if (fr) v1 = -v1;
+  if (r.fr) v1 = -v1;
   if (ii < 0 && a.bc[0] == BC_WIND_INNER) v1 = dmin(v1, 0.0);
-  if (ft) v2 = -v2;
+  if (r.ft) v2 = -v2;
 }
 
 // VGradCalc for one cell (line_connect.c:628-738) from the stage input:
@@ -221,14 +234,17 @@ struct VGrad {
   double x, z, maxds, x11_0, dx0, rdx0;   // rdx0 = 1 / dx0 for div_rc
 };
 
-__device__ __forceinline__ void vgrad_cell(const StageArgs& a, int j, int i, VGrad& g) {
+// R[dj][di]: the velocities of (j+dj-1, i+di-1) as loaded.
+__device__ __forceinline__ void vgrad_cell(const StageArgs& a, int j, int i,
+                                           const RawVel (&R)[3][3], VGrad& g) {
   const Const& k = a.k;
   const Tables& T = a.T;
   double P1[3][3], P2[3][3];
 #pragma unroll
   for (int dj = 0; dj < 3; dj++)
 #pragma unroll
-    for (int di = 0; di < 3; di++) ld_vel(a, j + dj - 1, i + di - 1, P1[dj][di], P2[dj][di]);
+    for (int di = 0; di < 3; di++)
+      vel_state(a, i + di - 1, R[dj][di], P1[dj][di], P2[dj][di]);
   // P[dj][di] = V(j+dj-1, i+di-1)
   g.v11_0 = (P1[0][0] + P1[0][1] + P1[1][0] + P1[1][1]) / 4.0;
   g.v11_1 = (P2[0][0] + P2[0][1] + P2[1][0] + P2[1][1]) / 4.0;
@@ -262,6 +278,15 @@ __device__ __forceinline__ void vgrad_cell(const StageArgs& a, int j, int i, VGr
   g.rdx0 = 1.0 / g.dx0;
   g.x = T.x1[I] * sj * UL;
   g.z = T.x1[I] * cj * UL;
+}
+
+__device__ __forceinline__ void vgrad_cell(const StageArgs& a, int j, int i, VGrad& g) {
+  RawVel R[3][3];
+#pragma unroll
+  for (int dj = 0; dj < 3; dj++)
+#pragma unroll
+    for (int di = 0; di < 3; di++) vel_issue(a, j + dj - 1, i + di - 1, R[dj][di]);
+  vgrad_cell(a, j, i, R, g);
 }
 
 // g2, so, co: the cell's LF_F2, LF_SIN and LF_COS entries of bin `ang`.
@@ -539,13 +564,29 @@ constexpr double LF_NUM_LO = 0x1p-100, LF_NUM_HI = 0x1p100;
 
 // The zone's part: both calls' num and the VGradCalc corners.
 template <int FEAT>
-__device__ __forceinline__ void lforce_zone(const StageArgs& a, int i, int j, LfCell& z) {
+__device__ __forceinline__ bool lforce_zone(const StageArgs& a, int i, int j, LfCell& z) {
   const Const& k = a.k;
   double vc[NVW], w1[NVW], e1[NVW], c[6], vpi[NVW], vmi[NVW];
-  ld6(a, a.Vin, j, i, vc);
-  ld6(a, j, i - 1, w1);
-  ld6(a, j, i + 1, e1);
+  // every load of the nine zones is under way before the first rule waits
+  // (128 x 64, where a wavefront has its SIMD to itself: 15.5 -> 13.6 us; no
+  // change at 512 x 256)
+  const int halted = a.loop ? a.s->halt : 0;
+  RawState raw[3];                     // (j, i - 1 .. i + 1)
+  RawVel R[3][3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) raw_issue(a, a.Vin, j, i + d - 1, raw[d]);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    vel_issue(a, j - 1, i + d - 1, R[0][d]);
+    vel_issue(a, j + 1, i + d - 1, R[2][d]);
+    R[1][d] = {raw[d].v[RHO], raw[d].v[VX1], raw[d].v[VX2], raw[d].im, raw[d].jm, raw[d].fr,
+               raw[d].ft};
+  }
   ldc(a.T.pr, a.nr, i + NG, c);
+  if (halted) return false;
+  raw_state(a, j, i, raw[1], vc);
+  raw_state(a, j, i - 1, raw[0], w1);
+  raw_state(a, j, i + 1, raw[2], e1);
   plm_zone<0, FEAT & FEAT_CHAR>(a, j, i, w1, vc, e1, c, vpi, vmi);
   const double r1 = 0.5 * (vpi[RHO] + vmi[RHO]), p1 = 0.5 * (vpi[PRS] + vmi[PRS]);
   const double rho1 = r1 * k.UD, rho2 = vc[RHO] * k.UD;
@@ -555,7 +596,8 @@ __device__ __forceinline__ void lforce_zone(const StageArgs& a, int i, int j, Lf
   const double vth2 = sqrt((2.0 * C_kB * T2) / C_mp);
   z.num1 = k.sigma_e * rho1 * vth1;
   z.num2 = k.sigma_e * rho2 * vth2;
-  vgrad_cell(a, j, i, z.vg);
+  vgrad_cell(a, j, i, R, z.vg);
+  return true;
 }
 
 // The zone's bins ang0, ang0 + step, ...: f(ang, g_r term, g_theta term);
@@ -1118,7 +1160,7 @@ template <int FEAT>
 __device__ __forceinline__ void lforce_zone_bins(const StageArgs& a, unsigned cell) {
   const int j = cell / (unsigned)a.nr, i = cell - j * a.nr;
   LfCell z;
-  lforce_zone<FEAT>(a, i, j, z);
+  if (!lforce_zone<FEAT>(a, i, j, z)) return;
   double g1r = 0.0, g2t = 0.0;
   lforce_bins(
       a, z, cell, 0, 1,
@@ -1138,7 +1180,6 @@ __device__ __forceinline__ void lforce_zone_bins(const StageArgs& a, unsigned ce
 template <int FEAT>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void wind_lforce_fast_kernel(StageArgs a) {
-  if (a.loop && a.s->halt) return;     // uniform over the launch
   const unsigned cell = blockIdx.x * 128 + threadIdx.x;
   if (cell < a.sv) lforce_zone_bins<FEAT>(a, cell);
 }
@@ -1149,14 +1190,14 @@ template <int FEAT, int S>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3)))
 void wind_lforce_split_kernel(StageArgs a) {
   extern __shared__ double terms[];    // [na][2][64]
-  if (a.loop && a.s->halt) return;     // uniform over the launch
   const unsigned cell = blockIdx.x * 64 + threadIdx.x;
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  bool live = false;                   // false: off the grid, or the run has stopped
   if (cell < a.sv) {
     const int j = cell / (unsigned)a.nr, i = cell - j * a.nr;
     LfCell z;
-    lforce_zone<FEAT>(a, i, j, z);
-    lforce_bins(
+    live = lforce_zone<FEAT>(a, i, j, z);
+    if (live) lforce_bins(
         a, z, cell, s, S,
         [&](int ang, double t1, double t2) {
           terms[(2 * ang) * 64 + threadIdx.x] = t1;
@@ -1165,7 +1206,7 @@ void wind_lforce_split_kernel(StageArgs a) {
         [] {});
   }
   __syncthreads();
-  if (cell < a.sv && s < 2) {
+  if (live && s < 2) {
     double sum = 0.0;
     for (int ang = 0; ang < a.na; ang++) sum += terms[(2 * ang + s) * 64 + threadIdx.x];
     a.glf[s * a.sv + cell] = sum;
@@ -1517,7 +1558,7 @@ int features(const pmx_wind* w) {
 }
 
 // Four wavefronts share the bins of 64 zones while the zones alone make
-// fewer than one and a half wavefronts per SIMD (8 k cells: 15 against 30 us,
+// fewer than one and a half wavefronts per SIMD (8 k cells: 14 against 30 us,
 // 43 k: 29 against 50, 74 k: 45 against 52, 98 k: 54 both ways, 131 k: 75
 // against 62; two or eight wavefronts measured slower from 20 k cells on).
 constexpr long long LF_SPLIT_CELLS = 3 * 64 * 1024 / 2;
