@@ -399,8 +399,8 @@ int advance(pmx_hydro* h, const double* dt_override, bool with_prep) {
 
 // Steps first .. first + n - 1 of a main-loop run.  A 2-D step is its stage
 // kernels alone: the time state alternates between s[0] and s[1], each
-// step's stage 1 ending the one before (KH 64^2: 6.4 -> 4.2 us per step,
-// whose launches take about 2 us each).
+// step's stage 1 ending the one before (KH 64^2: 17.6 -> 13.4 us per step, with
+// three runs side by side on streams of their own 6.4 -> 4.9).
 int run_steps(pmx_hydro* h, int first, int n) {
   for (int q = first; q < first + n; q++) {
     if (h->d.dims == 2) {

@@ -548,8 +548,8 @@ __device__ __forceinline__ void lforce_cell(const StageArgs& a, int i, int j) {
 // instructions, 267 per bin against 445 of lforce_cell: quotients and roots
 // without scaling, reciprocals shared, the root's serving the division by
 // ds, one straight-line block for both powers, coefficients in scalar
-// registers.  512 x 256: 89 -> 62 us per launch (24.8 M instead of 32.8 M
-// wave instructions at the first of its steps, 21.5 M now).
+// registers.  512 x 256: 89 -> 62 us per launch (55 over the first steps of a
+// run, when fewer bins see a gradient).
 // dvds is range-checked over the loop; a zone with one outside (or with such
 // a num) takes its bins again in the general form.
 // ---------------------------------------------------------------------
