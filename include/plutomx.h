@@ -82,8 +82,9 @@ typedef struct {
 
 const char *pmx_last_error(void);
 
-/* Create a context: allocates V (3 buffers), U and the grid tables on the
- * current HIP device.  Replaces the reference's one-time set-up in
+/* Create a context: allocates V (3 buffers; the second at least as long as
+ * a ghosted Vc of up to 32 MiB), U and the grid tables on the current HIP
+ * device.  Replaces the reference's one-time set-up in
  * Initialize() (Src/initialize.c:381-443) for the hot path. */
 int pmx_hydro_create(const pmx_hydro_desc *desc, pmx_hydro **out);
 int pmx_hydro_destroy(pmx_hydro *h);
@@ -91,7 +92,9 @@ int pmx_hydro_destroy(pmx_hydro *h);
 /* Host <-> device transfer of the primitive state Vc.  ghosts != 0 means
  * the host array is PLUTO's Vc[nv][NX3_TOT][NX2_TOT][NX1_TOT] with
  * nghost ghost cells in every active direction (Src/initialize.c:442);
- * on download the ghost cells are filled by the boundary rule. */
+ * on download the ghost cells are filled by the boundary rule.  Ghosted
+ * and interleaved arrays pass through the context's stage buffer in
+ * pieces: no transfer allocates device memory. */
 int pmx_hydro_set_prim(pmx_hydro *h, const double *V, int ghosts);
 int pmx_hydro_get_prim(pmx_hydro *h, double *V, int ghosts);
 /* Download Uc after the last stage.  pluto_layout != 0 writes the

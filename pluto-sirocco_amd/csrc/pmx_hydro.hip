@@ -72,55 +72,70 @@ __global__ __launch_bounds__(64) void finish_run_kernel(DevScalars* s, int which
 }
 
 // PLUTO's ghosted Vc[nv][k][j][i] from / to the interior arrays, the ghost
-// cells filled by the boundary rules, and its Uc[cell][nv] from U.  The
-// host's transfers are then of arrays as PLUTO holds them; these passes run
-// at HBM speed (14 MB, 64^3: a few us) where loops over the host arrays took
-// 3.8 ms of a 64^3 step's download and 0.4 ms of its upload.
+// cells filled by the boundary rules, and its Uc[cell][nv] from U: values
+// q0 .. q0 + m of PLUTO's array from / to a buffer.  The host's transfers are
+// then of arrays as PLUTO holds them; these passes run at HBM speed (14 MB,
+// 64^3: a few us) where loops over the host arrays took 3.8 ms of a 64^3
+// step's download and 0.4 ms of its upload.
 struct GhostLayout {
   int nx, ny, nz, g[3];          // interior, ghost cells per direction
   int bc[6];
   __host__ __device__ long long tx() const { return nx + 2 * g[0]; }
   __host__ __device__ long long ty() const { return ny + 2 * g[1]; }
   __host__ __device__ long long tz() const { return nz + 2 * g[2]; }
+  __host__ __device__ long long cells() const { return tx() * ty() * tz(); }
 };
 
-__global__ __launch_bounds__(256) void ghost_pack_kernel(const double* __restrict__ V,
-                                                         double* __restrict__ G, GhostLayout L) {
-  const long long n = L.tx() * L.ty() * L.tz(), sv = (long long)L.nx * L.ny * L.nz;
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int i = (int)(q % L.tx()), j = (int)(q / L.tx() % L.ty()), k = (int)(q / L.tx() / L.ty());
-  bool fx = false, fy = false, fz = false;
-  const int ii = map_bc(i - L.g[0], L.nx, L.bc[0], L.bc[1], fx);
-  const int jj = map_bc(j - L.g[1], L.ny, L.bc[2], L.bc[3], fy);
-  const int kk = L.g[2] ? map_bc(k - L.g[2], L.nz, L.bc[4], L.bc[5], fz) : 0;
-  const double* p = V + ((long long)kk * L.ny + jj) * L.nx + ii;
-  double v[NV];
-#pragma unroll
-  for (int nv = 0; nv < NV; nv++) v[nv] = p[nv * sv];
-  if (fx) v[VX1] = -v[VX1];
-  if (fy) v[VX2] = -v[VX2];
-  if (fz) v[VX3] = -v[VX3];
-#pragma unroll
-  for (int nv = 0; nv < NV; nv++) G[nv * n + q] = v[nv];
+// Variable and indices of value q of the ghosted array.
+struct GhostIndex {
+  int nv, i, j, k;
+};
+__device__ __forceinline__ GhostIndex ghost_index(const GhostLayout& L, long long q) {
+  GhostIndex x;
+  const long long n = L.cells();
+  x.nv = (int)(q / n);
+  const unsigned tx = (unsigned)L.tx(), ty = (unsigned)L.ty();
+  long long r = q - x.nv * n;
+  x.i = (int)(r % tx);
+  r /= tx;
+  x.j = (int)(r % ty);
+  x.k = (int)(r / ty);
+  return x;
 }
 
-__global__ __launch_bounds__(256) void ghost_unpack_kernel(const double* __restrict__ G,
-                                                           double* __restrict__ V, GhostLayout L) {
-  const long long n = L.tx() * L.ty() * L.tz(), sv = (long long)L.nx * L.ny * L.nz;
+__global__ __launch_bounds__(256) void ghost_pack_kernel(const double* __restrict__ V,
+                                                         double* __restrict__ buf, GhostLayout L,
+                                                         long long q0, long long m) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= sv) return;
-  const int i = (int)(q % L.nx), j = (int)(q / L.nx % L.ny), k = (int)(q / L.nx / L.ny);
-  const double* p = G + ((k + L.g[2]) * L.ty() + j + L.g[1]) * L.tx() + i + L.g[0];
-#pragma unroll
-  for (int nv = 0; nv < NV; nv++) V[nv * sv + q] = p[nv * n];
+  if (q >= m) return;
+  const GhostIndex x = ghost_index(L, q0 + q);
+  bool flip[3] = {false, false, false};
+  const int i = map_bc(x.i - L.g[0], L.nx, L.bc[0], L.bc[1], flip[0]);
+  const int j = map_bc(x.j - L.g[1], L.ny, L.bc[2], L.bc[3], flip[1]);
+  const int k = L.g[2] ? map_bc(x.k - L.g[2], L.nz, L.bc[4], L.bc[5], flip[2]) : 0;
+  const double v = V[(((long long)x.nv * L.nz + k) * L.ny + j) * L.nx + i];
+  const bool neg = (x.nv == VX1 && flip[0]) || (x.nv == VX2 && flip[1]) ||
+                   (x.nv == VX3 && flip[2]);
+  buf[q] = neg ? -v : v;
+}
+
+__global__ __launch_bounds__(256) void ghost_unpack_kernel(const double* __restrict__ buf,
+                                                           double* __restrict__ V, GhostLayout L,
+                                                           long long q0, long long m) {
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= m) return;
+  const GhostIndex x = ghost_index(L, q0 + q);
+  const int i = x.i - L.g[0], j = x.j - L.g[1], k = x.k - L.g[2];
+  if (i >= 0 && i < L.nx && j >= 0 && j < L.ny && k >= 0 && k < L.nz)
+    V[(((long long)x.nv * L.nz + k) * L.ny + j) * L.nx + i] = buf[q];
 }
 
 __global__ __launch_bounds__(256) void cons_interleave_kernel(const double* __restrict__ U,
-                                                              double* __restrict__ out,
-                                                              long long ncell) {
+                                                              double* __restrict__ buf,
+                                                              long long ncell, long long q0,
+                                                              long long m) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < NV * ncell) out[q] = U[q % NV * ncell + q / NV];
+  if (q < m) buf[q] = U[(q0 + q) % NV * ncell + (q0 + q) / NV];
 }
 
 // Plain streaming copy, used to calibrate the HBM byte counters and to
@@ -155,8 +170,7 @@ struct pmx_hydro {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pending;
   double timed_ms;
   int timed_launches;
-  double* gbuf;     // hand-over arrays in PLUTO's layouts, from their first use on
-  size_t gbuf_n;
+  long long piece;  // values of PLUTO's arrays handed over at a time, through V[1]
 };
 
 namespace {
@@ -445,18 +459,26 @@ GhostLayout ghost_layout(const pmx_hydro* h) {
   return L;
 }
 
-// The hand-over buffer, of at least n doubles.
-int ensure_gbuf(pmx_hydro* h, size_t n) {
-  if (h->gbuf_n >= n) return 0;
-  if (h->gbuf) PMX_HIP_CHECK(hipFree(h->gbuf));
-  h->gbuf = nullptr;
-  h->gbuf_n = 0;
-  PMX_HIP_CHECK(hipMalloc(&h->gbuf, sizeof(double) * n));
-  h->gbuf_n = n;
-  return 0;
+// PLUTO's arrays are handed over in pieces through V[1], which holds nothing
+// between two steps, so a hand-over needs no memory of its own.  V[1] is made
+// long enough that a ghosted array of up to HANDOVER_MIN values goes in one
+// piece (64^3: 1.7 M values, a step with both transfers 2.05 ms); a piece is
+// at most HANDOVER_MAX values, a launch of one thread each.
+constexpr long long HANDOVER_MIN = 1ll << 22, HANDOVER_MAX = 1ll << 28;
+
+long long handover_values(const pmx_hydro* h) {
+  return std::max(NV * h->ncell, std::min(NV * ghost_layout(h).cells(), HANDOVER_MIN));
 }
 
 unsigned blocks256(long long n) { return (unsigned)((n + 255) / 256); }
+
+// f(q0, m) for the pieces of an array of n values
+template <class F>
+int by_pieces(const pmx_hydro* h, long long n, F f) {
+  for (long long q0 = 0; q0 < n; q0 += h->piece)
+    if (f(q0, std::min(h->piece, n - q0))) return -1;
+  return 0;
+}
 
 // The checks pmx_hydro_create makes of a descriptor.
 int check_desc(const pmx_hydro_desc* desc) {
@@ -515,7 +537,9 @@ int pmx_hydro_create(const pmx_hydro_desc* desc, pmx_hydro** out) {
 #define CK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { \
     set_error(std::string(#x) + ": " + hipGetErrorString(e_)); pmx_hydro_destroy(h); return -1; } } while (0)
   CK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
-  for (int q = 0; q < 3; q++) CK(hipMalloc(&h->V[q], vbytes));
+  const long long held = handover_values(h);
+  h->piece = std::min(held, HANDOVER_MAX);
+  for (int q = 0; q < 3; q++) CK(hipMalloc(&h->V[q], q == 1 ? sizeof(double) * held : vbytes));
   CK(hipMalloc(&h->U, vbytes));
   CK(hipMalloc(&h->dx, sizeof(double) * ntot));
   CK(hipMalloc(&h->dtdx, sizeof(double) * ntot));
@@ -551,7 +575,6 @@ int pmx_hydro_destroy(pmx_hydro* h) {
   if (h->inv_dl) hipFree(h->inv_dl);
   if (h->s) hipFree(h->s);
   if (h->dt_in) hipFree(h->dt_in);
-  if (h->gbuf) hipFree(h->gbuf);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;
   return 0;
@@ -559,19 +582,19 @@ int pmx_hydro_destroy(pmx_hydro* h) {
 
 int pmx_hydro_set_prim(pmx_hydro* h, const double* V, int ghosts) {
   if (!h || !V) { set_error("null argument"); return -1; }
-  const size_t n = (size_t)NV * h->ncell;
   if (ghosts) {
     const GhostLayout L = ghost_layout(h);
-    const size_t ng = (size_t)NV * L.tx() * L.ty() * L.tz();
-    if (ensure_gbuf(h, ng)) return -1;
-    PMX_HIP_CHECK(hipMemcpyAsync(h->gbuf, V, ng * sizeof(double), hipMemcpyHostToDevice,
-                                 h->stream));
-    hipLaunchKernelGGL(ghost_unpack_kernel, dim3(blocks256(h->ncell)), dim3(256), 0, h->stream,
-                       h->gbuf, h->V[0], L);
-    PMX_HIP_CHECK(hipGetLastError());
+    if (by_pieces(h, NV * L.cells(), [&](long long q0, long long m) {
+          PMX_HIP_CHECK(hipMemcpyAsync(h->V[1], V + q0, m * sizeof(double), hipMemcpyHostToDevice,
+                                       h->stream));
+          hipLaunchKernelGGL(ghost_unpack_kernel, dim3(blocks256(m)), dim3(256), 0, h->stream,
+                             h->V[1], h->V[0], L, q0, m);
+          PMX_HIP_CHECK(hipGetLastError());
+          return 0;
+        })) return -1;
   } else {
-    PMX_HIP_CHECK(hipMemcpyAsync(h->V[0], V, n * sizeof(double), hipMemcpyHostToDevice,
-                                 h->stream));
+    PMX_HIP_CHECK(hipMemcpyAsync(h->V[0], V, sizeof(double) * NV * h->ncell,
+                                 hipMemcpyHostToDevice, h->stream));
   }
   PMX_HIP_CHECK(hipStreamSynchronize(h->stream));
   return 0;
@@ -579,35 +602,39 @@ int pmx_hydro_set_prim(pmx_hydro* h, const double* V, int ghosts) {
 
 int pmx_hydro_get_prim(pmx_hydro* h, double* V, int ghosts) {
   if (!h || !V) { set_error("null argument"); return -1; }
-  size_t n = (size_t)NV * h->ncell;
-  const double* src = h->V[0];
   if (ghosts) {
     const GhostLayout L = ghost_layout(h);
-    const long long cells = L.tx() * L.ty() * L.tz();
-    n = (size_t)NV * cells;
-    if (ensure_gbuf(h, n)) return -1;
-    hipLaunchKernelGGL(ghost_pack_kernel, dim3(blocks256(cells)), dim3(256), 0, h->stream,
-                       h->V[0], h->gbuf, L);
-    PMX_HIP_CHECK(hipGetLastError());
-    src = h->gbuf;
+    if (by_pieces(h, NV * L.cells(), [&](long long q0, long long m) {
+          hipLaunchKernelGGL(ghost_pack_kernel, dim3(blocks256(m)), dim3(256), 0, h->stream,
+                             h->V[0], h->V[1], L, q0, m);
+          PMX_HIP_CHECK(hipGetLastError());
+          PMX_HIP_CHECK(hipMemcpyAsync(V + q0, h->V[1], m * sizeof(double),
+                                       hipMemcpyDeviceToHost, h->stream));
+          return 0;
+        })) return -1;
+  } else {
+    PMX_HIP_CHECK(hipMemcpyAsync(V, h->V[0], sizeof(double) * NV * h->ncell,
+                                 hipMemcpyDeviceToHost, h->stream));
   }
-  PMX_HIP_CHECK(hipMemcpyAsync(V, src, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   PMX_HIP_CHECK(hipStreamSynchronize(h->stream));
   return 0;
 }
 
 int pmx_hydro_get_cons(pmx_hydro* h, double* U, int pluto_layout) {
   if (!h || !U) { set_error("null argument"); return -1; }
-  const size_t n = (size_t)NV * h->ncell;
-  const double* src = h->U;
   if (pluto_layout) {
-    if (ensure_gbuf(h, n)) return -1;
-    hipLaunchKernelGGL(cons_interleave_kernel, dim3(blocks256((long long)n)), dim3(256), 0,
-                       h->stream, h->U, h->gbuf, h->ncell);
-    PMX_HIP_CHECK(hipGetLastError());
-    src = h->gbuf;
+    if (by_pieces(h, NV * h->ncell, [&](long long q0, long long m) {
+          hipLaunchKernelGGL(cons_interleave_kernel, dim3(blocks256(m)), dim3(256), 0, h->stream,
+                             h->U, h->V[1], h->ncell, q0, m);
+          PMX_HIP_CHECK(hipGetLastError());
+          PMX_HIP_CHECK(hipMemcpyAsync(U + q0, h->V[1], m * sizeof(double),
+                                       hipMemcpyDeviceToHost, h->stream));
+          return 0;
+        })) return -1;
+  } else {
+    PMX_HIP_CHECK(hipMemcpyAsync(U, h->U, sizeof(double) * NV * h->ncell, hipMemcpyDeviceToHost,
+                                 h->stream));
   }
-  PMX_HIP_CHECK(hipMemcpyAsync(U, src, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   PMX_HIP_CHECK(hipStreamSynchronize(h->stream));
   return 0;
 }
