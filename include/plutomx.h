@@ -573,6 +573,25 @@ int pmx_check_div_rc(const double *x, long long n, double c, long long *mismatch
 int pmx_check_force_power(const double *num, const double *dvds, long long n, double krad,
                           double alpha, double *out);
 
+/* Arithmetic check (no counterpart in the reference): n cells through the
+ * plain cooling integrator (cv_idl/cooling_source.c) with its short
+ * operations, with the general ones, and as CoolingSource takes them, on the
+ * device or (on_device 0) on the host.  desc: the scalars of the wind; cell
+ * i has density rho, pressure p, ionisation parameter xi, step dt, the
+ * tracer open, prefactors pre[q * n + i] (comp_h, comp_c, xray_h, brem_c,
+ * line_c; NULL: 1).  Returns the first rate, the integrated energies e [2][n]
+ * (short, general), the new pressures p_out [2][n] (general, as taken), the
+ * Radiat() calls [3][n] (short, general, as taken) and the flags below; a
+ * cell without PMX_COOL_SHORT has no short energy (0). */
+#define PMX_COOL_SHORT       1   /* the short operations are tried */
+#define PMX_COOL_OVER        2   /* an energy left their range: done again */
+#define PMX_COOL_BAD_SHORT   4   /* sub-step limit reached: short, general, as taken */
+#define PMX_COOL_BAD_GENERAL 8
+#define PMX_COOL_BAD_TAKEN  16
+int pmx_check_cooling(const pmx_wind_desc *desc, int on_device, long long n, const double *rho,
+                      const double *p, const double *xi, const double *dt, const double *pre,
+                      double *rate, double *e, double *p_out, long long *calls, int *flags);
+
 #ifdef __cplusplus
 }
 #endif

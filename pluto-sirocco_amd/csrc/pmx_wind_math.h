@@ -768,8 +768,8 @@ PMX_HD void rad_prepare(const Const& k, RadCell& R) {
   R.rsqxi = recip(R.sqxi);
 }
 
-// Largest energy of radiat<true>; a cell that exceeds it is done again with
-// the general operations.
+// Largest energy, and trial energy of either sign, of radiat<true>; a cell
+// that exceeds it is done again with the general operations.
 constexpr double RAD_E_MAX = 0x1p300;
 
 // a / b, by the moderate quotient where MOD
@@ -786,15 +786,18 @@ PMX_HD double mdiv(double a, double b) {
 // and its root what moderate operands do not need and shares the
 // reciprocals (rho's and sqrt(xi)'s from rad_prepare, T's three times):
 // about 115 instructions instead of 180, the same bits.  For a cell with
-// R.moderate and E <= RAD_E_MAX (`over` tells): then T >= 1e4 K from here on
-// bounds every other operand.
+// R.moderate whose energies as given, before the floor, stay within
+// RAD_E_MAX (`over` tells).  T >= 1e4 K then bounds the operands from the
+// cut on, and the trial energies E0 + c dt k1 bound the integrators' error
+// scale |E0| + dt |k1| by 2^304.  Below, that scale is E0, which is at least
+// 2^-300 to begin with: a later one is 0 or a multiple of its last bits.
 template <bool MOD = false>
 PMX_HD double radiat(const Const& k, const RadCell& R, double& E, bool& over) {
   const double minT = 1.e4;
   R.nev++;
+  if (MOD) over = over | !(fabs(E) <= RAD_E_MAX);
   double prs = E * (k.gamma - 1.0);
   if (prs < 0.0) { prs = 1.e-12; E = prs / (k.gamma - 1.0); }
-  if (MOD) over = over | !(E <= RAD_E_MAX);
   double T = (MOD ? quot(prs, R.rho, R.rrho) : prs / R.rho) * k.KELVIN * k.mu;
   if (T < minT) return 0.0;
   const double nH = R.nH, xi = R.xi, tx = R.tx, sqxi = R.sqxi, sqsqxi = R.sqsqxi;
@@ -952,6 +955,11 @@ PMX_HD double integrate_cell(const Const& k, const RadCell& R, double dt, double
   return E1;
 }
 
+// Whether a cell is given to the short operations.
+PMX_HD bool short_form(const RadCell& R, double E0, double dt) {
+  return R.moderate && in_range(E0, 0x1p-300, RAD_E_MAX) && in_range(dt, 0x1p-300, 0x1p300);
+}
+
 // One cell of CoolingSource: returns the new pressure and the cell's
 // dt * maxCoolingRate / |dp/p| candidate for dt_cool, from a first rate
 // already formed.  A cell of moderate state takes the short operations, and
@@ -959,8 +967,7 @@ PMX_HD double integrate_cell(const Const& k, const RadCell& R, double dt, double
 PMX_HD double plain_cell_from(const Const& k, const RadCell& R, double p, double dt, double E0,
                               double k1, double& dt_cool_cell, int& bad) {
   const int nev = R.nev;
-  bool general = !(R.moderate && in_range(E0, 0x1p-300, RAD_E_MAX) &&
-                   in_range(dt, 0x1p-300, 0x1p300));
+  bool general = !short_form(R, E0, dt);
   double E1 = E0;
   int b = 0;
   if (!general) E1 = integrate_cell<true>(k, R, dt, E0, k1, b, general);

@@ -34,7 +34,7 @@ EXPORTS = ["pmx_last_error", "pmx_hydro_create", "pmx_hydro_destroy", "pmx_hydro
            "pmx_hydro_get_time", "pmx_hydro_advance_step", "pmx_hydro_run",
            "pmx_hydro_sync", "pmx_hydro_run_graph", "pmx_hydro_stage_timing",
            "pmx_hydro_device_state", "pmx_copy_probe", "pmx_copy_probe_runtime", "pmx_check_div_rc",
-           "pmx_check_force_power",
+           "pmx_check_force_power", "pmx_check_cooling",
            "pmx_wind_create", "pmx_wind_destroy", "pmx_wind_set_prim", "pmx_wind_get_prim",
            "pmx_wind_get_cons", "pmx_wind_set_heatcool", "pmx_wind_set_time",
            "pmx_wind_get_time", "pmx_wind_set_dts", "pmx_wind_advance_step", "pmx_wind_split_source",
@@ -143,6 +143,8 @@ def load_library(path: pathlib.Path | str | None = None) -> ctypes.CDLL:
                                       ctypes.POINTER(ctypes.c_longlong)]
     lib.pmx_check_force_power.argtypes = [dp, dp, ctypes.c_longlong, ctypes.c_double,
                                           ctypes.c_double, dp]
+    lib.pmx_check_cooling.argtypes = [ctypes.POINTER(WindDesc), ctypes.c_int, ctypes.c_longlong,
+                                      *[dp] * 8, ctypes.POINTER(ctypes.c_longlong), ip]
     lp = ctypes.POINTER(ctypes.c_long)
     lib.pmx_wind_create.argtypes = [ctypes.POINTER(WindDesc), ctypes.POINTER(vp)]
     lib.pmx_wind_destroy.argtypes = [vp]
@@ -256,6 +258,27 @@ def check_force_power(num: np.ndarray, dvds: np.ndarray, krad: float, alpha: flo
     _check(load_library().pmx_check_force_power(_dptr(num), _dptr(dvds), num.size, float(krad),
                                                 float(alpha), _dptr(out)), "check_force_power")
     return out
+
+
+def check_cooling(cfg: setups.WindConfig, rho, p, xi, dt, pre=None, device: bool = True) -> dict:
+    """Cells through the plain cooling integrator with its short operations,
+    with the general ones and as CoolingSource takes them (include/plutomx.h,
+    pmx_check_cooling); pre: (5, n) prefactors."""
+    arrs = [np.ascontiguousarray(a, dtype=np.float64) for a in (rho, p, xi, dt)]
+    n = arrs[0].size
+    if any(a.shape != (n,) for a in arrs) or (pre is not None and np.shape(pre) != (5, n)):
+        raise ValueError("the cells' arrays differ in shape")
+    pre = None if pre is None else np.ascontiguousarray(pre, dtype=np.float64)
+    d = wind_desc_scalars(cfg)
+    rate, e, pn = np.empty(n), np.empty((2, n)), np.empty((2, n))
+    calls, flags = np.empty((3, n), dtype=np.int64), np.empty(n, dtype=np.intc)
+    _check(load_library().pmx_check_cooling(
+        ctypes.byref(d), int(device), n, *map(_dptr, arrs), None if pre is None else _dptr(pre),
+        _dptr(rate), _dptr(e), _dptr(pn),
+        calls.ctypes.data_as(ctypes.POINTER(ctypes.c_longlong)),
+        flags.ctypes.data_as(ctypes.POINTER(ctypes.c_int))), "check_cooling")
+    return {"rate": rate, "e": e, "p": pn, "calls": calls, "short": flags & 1 != 0,
+            "over": flags & 2 != 0, "bad": np.array([flags & b != 0 for b in (4, 8, 16)])}
 
 
 def copy_probe(nbytes: int, reps: int = 10, runtime: bool = False) -> float:
