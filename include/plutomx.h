@@ -565,13 +565,32 @@ int pmx_check_div_rc(const double *x, long long n, double c, long long *mismatch
 
 /* Arithmetic check (no counterpart in the reference): the line force's
  * force-multiplier power M = krad pow(t, alpha), t = num / dvds
- * (Src/LineDriven/line_connect.c:880-881), as the device evaluates it:
- * log2 num per LineForce call and log2 dvds per bin, shared, in
- * double-double, and 2^(alpha log2 t) with the quotient's rounding error
- * folded in.  out[i] = krad pow(num[i] / dvds[i], alpha) for dvds[i] > 0,
- * else 0 (host arrays of n values). */
+ * (Src/LineDriven/line_connect.c:880-881), as the device evaluates it in
+ * its general form: log2 num per LineForce call and log2 dvds per bin,
+ * shared, in double-double, and 2^(alpha log2 t) with the quotient's
+ * rounding error folded in.  out[i] = krad pow(num[i] / dvds[i], alpha) for
+ * dvds[i] > 0, else 0 (host arrays of n values).  The form for operands of
+ * moderate exponent: pmx_check_force_mult. */
 int pmx_check_force_power(const double *num, const double *dvds, long long n, double krad,
                           double alpha, double *out);
+
+/* Arithmetic check (no counterpart in the reference): of the n pairs (x, c),
+ * |x|, |c| and |x / c| within 2^-900..2^900, how many quotients x / c by the
+ * quotient with a reciprocal of its own (mismatches[0]) and by the one whose
+ * divisor many share (mismatches[1]), and how many roots of |x|
+ * (mismatches[2]), differ from the device's general operations in value (0
+ * expected). */
+int pmx_check_quotients(const double *x, const double *c, long long n, long long *mismatches);
+
+/* Arithmetic check (no counterpart in the reference): the force multiplier
+ * in the short form that the line force takes for operands of moderate
+ * exponent (num within 2^-100..2^100, dvds within 2^-400..2^400 or 0,
+ * |alpha| <= 2, krad >= 0), and in the general one.  out is [4][n]: the
+ * power krad pow(num / dvds, alpha) and the capped M of the short form (the
+ * power means nothing where dvds is 0 or NaN), then both of the general
+ * form. */
+int pmx_check_force_mult(const double *num, const double *dvds, long long n, double krad,
+                         double alpha, double *out);
 
 /* Arithmetic check (no counterpart in the reference): n cells through the
  * plain cooling integrator (cv_idl/cooling_source.c) with its short

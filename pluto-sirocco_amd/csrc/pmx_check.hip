@@ -1,7 +1,9 @@
-// Arithmetic check: the short operations of the plain cooling integrator
-// beside the general ones, on the same cells.  It calls the functions the
-// kernels call, from a translation unit of its own, so that the kernels'
-// inlining does not depend on it.
+// Arithmetic checks: the short operations of the Cartesian faces, the plain
+// cooling integrator and the line force beside the general ones, on the same
+// operands.  They call the functions the kernels call, from a translation
+// unit of their own, so that the kernels' inlining does not depend on them.
+#include <algorithm>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -37,6 +39,47 @@ struct DeviceArrays {
     return -1;
   }
 };
+
+dim3 blocks(long long n) { return dim3((unsigned)std::min<long long>((n + 255) / 256, 4096)); }
+
+// ---------------------------------------------------------------------
+// quotients and roots
+// ---------------------------------------------------------------------
+__global__ void quotient_check_kernel(const double* __restrict__ x, const double* __restrict__ c,
+                                      long long n, unsigned long long* bad) {
+  unsigned long long mine[3] = {0, 0, 0};
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const double a = x[i], b = c[i], r = a / b, s = fabs(a);
+    mine[0] += quot(a, b, recip(b)) != r;
+    mine[1] += div2(a, recip2(b, 1.0 / b)) != r;
+    double y;
+    mine[2] += s > 0.0 && sqrt_mod(s, y) != sqrt(s);
+  }
+  for (int q = 0; q < 3; q++)
+    if (mine[q]) atomicAdd(bad + q, mine[q]);
+}
+
+// ---------------------------------------------------------------------
+// force multiplier
+// ---------------------------------------------------------------------
+// out: [power, M] of the short form, [power, M] of the general one
+__global__ void force_check_kernel(const double* __restrict__ num, const double* __restrict__ dvds,
+                                   long long n, Const k, double* __restrict__ out) {
+  const PowSeries C = pow_series();
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
+       i += (long long)gridDim.x * blockDim.x) {
+    const double d = dvds[i], y = recip(d);
+    int e;
+    const PowNum a = pow_num_fast(num[i], C);
+    const DD D = log2_dd_fast(d, C, e);
+    out[i] = force_power_fast(k, a, d, y, D, C);
+    out[n + i] = force_mult_fast(k, a, d, y, D, C);
+    const double g = d > 0.0 ? force_power_shared(k, pow_num(num[i]), d, log2_dd(d)) : 0.0;
+    out[2 * n + i] = g;
+    out[3 * n + i] = g > 4400. ? 4400. : g;
+  }
+}
 
 // ---------------------------------------------------------------------
 // plain cooling integrator
@@ -101,6 +144,36 @@ using namespace pmx;
 using namespace pmx::wind;
 
 extern "C" {
+
+int pmx_check_quotients(const double* x, const double* c, long long n, long long* mismatches) {
+  if (!x || !c || n <= 0 || !mismatches) { set_error("bad argument"); return -1; }
+  DeviceArrays d;
+  unsigned long long bad[3] = {0, 0, 0};
+  const double *dx = d.make(x, n), *dc = d.make(c, n);
+  unsigned long long* db = d.make(bad, 3);
+  if (d.result()) return -1;
+  hipLaunchKernelGGL(quotient_check_kernel, blocks(n), dim3(256), 0, 0, dx, dc, n, db);
+  d.err = hipGetLastError();
+  d.read(bad, db, 3);
+  for (int q = 0; q < 3; q++) mismatches[q] = (long long)bad[q];
+  return d.result();
+}
+
+int pmx_check_force_mult(const double* num, const double* dvds, long long n, double krad,
+                         double alpha, double* out) {
+  if (!num || !dvds || n <= 0 || !out) { set_error("bad argument"); return -1; }
+  Const k{};
+  k.krad = krad;
+  k.alpharad = alpha;
+  DeviceArrays d;
+  const double *dn = d.make(num, n), *dd = d.make(dvds, n);
+  double* o = d.make((const double*)nullptr, 4 * n);
+  if (d.result()) return -1;
+  hipLaunchKernelGGL(force_check_kernel, blocks(n), dim3(256), 0, 0, dn, dd, n, k, o);
+  d.err = hipGetLastError();
+  d.read(out, o, 4 * n);
+  return d.result();
+}
 
 int pmx_check_cooling(const pmx_wind_desc* desc, int on_device, long long n, const double* rho,
                       const double* p, const double* xi, const double* dt, const double* pre,

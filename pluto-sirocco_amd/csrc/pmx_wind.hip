@@ -539,10 +539,11 @@ __device__ __forceinline__ void lforce_cell(const StageArgs& a, int i, int j) {
 }
 
 // ---------------------------------------------------------------------
-// The same line force, bit for bit (see force_mult_fast), for grids whose
-// inputs keep the operands' exponents moderate (k.lf_fast, decided at
-// create: the reference's power with |alpha| <= 2 and krad >= 0, fluxes,
-// radii and offset lengths within the ranges stated there).  The bin loop is
+// The same line force (the same bits but for the rare last one of a power,
+// see log2_dd_fast's section) for grids whose inputs keep the operands'
+// exponents moderate (k.lf_fast, decided at create: the reference's power
+// with |alpha| <= 2 and krad >= 0, fluxes, radii and offset lengths within
+// the ranges stated there).  The bin loop is
 // bound by VALU issue: two wavefronts per SIMD fill it, one by itself waits
 // twice as long for its own results.  This form is the one with few
 // instructions, 267 per bin against 445 of lforce_cell: quotients and roots
@@ -622,14 +623,7 @@ __device__ __forceinline__ void lforce_bins(const StageArgs& a, const LfCell& z,
                z.num2 <= LF_NUM_HI);
   {
     const PowSeries C = pow_series();
-    PowNum P[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      int n;
-      P[q].num = q ? z.num2 : z.num1;
-      P[q].rn = LOG2E_HI / P[q].num;
-      P[q].L = log2_dd_fast(P[q].num, C, n);
-    }
+    const PowNum P[2] = {pow_num_fast(z.num1, C), pow_num_fast(z.num2, C)};
     const Recip2 dx0 = recip2(g.dx0, g.rdx0), rc = recip2(C_c, 1.0 / C_c),
                  ua = recip2(k.UA, 1.0 / k.UA);
     double dmax_ = 0.0;                  // largest dvds, and the smallest's scaling
@@ -1739,9 +1733,9 @@ __global__ void div_check_kernel(const double* __restrict__ x, long long n, doub
   if (mine) atomicAdd(bad, mine);
 }
 
-// The line force's reference-form power krad pow(num / dvds, alpha) as the
-// line-force kernel evaluates it (force_power_shared), per element; 0 where
-// dvds <= 0 (a bin the reference leaves at M = 0).
+// The line force's reference-form power krad pow(num / dvds, alpha) in the
+// general form (force_power_shared), per element; 0 where dvds <= 0 (a bin
+// the reference leaves at M = 0).
 __global__ void power_check_kernel(const double* __restrict__ num, const double* __restrict__ dvds,
                                    long long n, Const k, double* __restrict__ out) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
@@ -1935,7 +1929,7 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
         maxds /= 2.0;
         double fr = d->flux_r[q], ft = d->flux_t[q], fp = d->flux_p[q];
         if (!div_rc_flux_ok(fr) || !div_rc_flux_ok(ft)) fast_div = false;
-        // the roots of lforce_cell_fast: the offset length and radius
+        // the roots of lforce_bins: the offset length and radius
         if (!(maxds >= 0x1p-300 && maxds <= 0x1p300)) lf_geom = false;
         double mod_flux = sqrt(pow(fr, 2) + pow(ft, 2) + pow(fp, 2));
         lf[LF_FR * sa + q] = fr;

@@ -34,7 +34,8 @@ EXPORTS = ["pmx_last_error", "pmx_hydro_create", "pmx_hydro_destroy", "pmx_hydro
            "pmx_hydro_get_time", "pmx_hydro_advance_step", "pmx_hydro_run",
            "pmx_hydro_sync", "pmx_hydro_run_graph", "pmx_hydro_stage_timing",
            "pmx_hydro_device_state", "pmx_copy_probe", "pmx_copy_probe_runtime", "pmx_check_div_rc",
-           "pmx_check_force_power", "pmx_check_cooling",
+           "pmx_check_force_power", "pmx_check_quotients", "pmx_check_force_mult",
+           "pmx_check_cooling",
            "pmx_wind_create", "pmx_wind_destroy", "pmx_wind_set_prim", "pmx_wind_get_prim",
            "pmx_wind_get_cons", "pmx_wind_set_heatcool", "pmx_wind_set_time",
            "pmx_wind_get_time", "pmx_wind_set_dts", "pmx_wind_advance_step", "pmx_wind_split_source",
@@ -143,6 +144,10 @@ def load_library(path: pathlib.Path | str | None = None) -> ctypes.CDLL:
                                       ctypes.POINTER(ctypes.c_longlong)]
     lib.pmx_check_force_power.argtypes = [dp, dp, ctypes.c_longlong, ctypes.c_double,
                                           ctypes.c_double, dp]
+    lib.pmx_check_quotients.argtypes = [dp, dp, ctypes.c_longlong,
+                                        ctypes.POINTER(ctypes.c_longlong)]
+    lib.pmx_check_force_mult.argtypes = [dp, dp, ctypes.c_longlong, ctypes.c_double,
+                                         ctypes.c_double, dp]
     lib.pmx_check_cooling.argtypes = [ctypes.POINTER(WindDesc), ctypes.c_int, ctypes.c_longlong,
                                       *[dp] * 8, ctypes.POINTER(ctypes.c_longlong), ip]
     lp = ctypes.POINTER(ctypes.c_long)
@@ -238,8 +243,10 @@ def cell_widths(cfg: setups.HydroConfig, d: int) -> np.ndarray:
 
 
 def check_div_rc(x: np.ndarray, c: float) -> int:
-    """Number of x whose device quotient x / c from the reciprocal-and-FMA
-    evaluation differs in any bit from the device division."""
+    """Number of x whose device quotient x / c in any of the short forms
+    (the constant divisor's, the one with a reciprocal of its own, the shared
+    one), or whose short root of |x|, differs from the device's division or
+    root.  check_quotients counts them one by one."""
     x = np.ascontiguousarray(x, dtype=np.float64)
     bad = ctypes.c_longlong()
     _check(load_library().pmx_check_div_rc(_dptr(x), x.size, float(c), ctypes.byref(bad)),
@@ -249,7 +256,8 @@ def check_div_rc(x: np.ndarray, c: float) -> int:
 
 def check_force_power(num: np.ndarray, dvds: np.ndarray, krad: float, alpha: float) -> np.ndarray:
     """The device's line-force power krad pow(num / dvds, alpha) per element
-    (0 where dvds <= 0), as the line-force kernel evaluates it."""
+    (0 where dvds <= 0) in its general form; check_force_mult has the short
+    one beside it."""
     num = np.ascontiguousarray(num, dtype=np.float64)
     dvds = np.ascontiguousarray(dvds, dtype=np.float64)
     if num.shape != dvds.shape:
@@ -258,6 +266,32 @@ def check_force_power(num: np.ndarray, dvds: np.ndarray, krad: float, alpha: flo
     _check(load_library().pmx_check_force_power(_dptr(num), _dptr(dvds), num.size, float(krad),
                                                 float(alpha), _dptr(out)), "check_force_power")
     return out
+
+
+def check_quotients(x: np.ndarray, c: np.ndarray) -> dict:
+    """How many of the pairs (x, c) have a device result that differs in value
+    from the general operation: x / c with a reciprocal of its own
+    ("quotient"), with a shared one ("shared"), and the root of |x| ("root")."""
+    x, c = (np.ascontiguousarray(a, dtype=np.float64) for a in (x, c))
+    if x.shape != c.shape:
+        raise ValueError("x and c differ in shape")
+    bad = (ctypes.c_longlong * 3)()
+    _check(load_library().pmx_check_quotients(_dptr(x), _dptr(c), x.size, bad),
+           "check_quotients")
+    return dict(zip(("quotient", "shared", "root"), bad))
+
+
+def check_force_mult(num: np.ndarray, dvds: np.ndarray, krad: float, alpha: float) -> dict:
+    """The line force's power krad pow(num / dvds, alpha) and its capped M in
+    the short form ("power", "M") and in the general one ("power_general",
+    "M_general"), per element."""
+    num, dvds = (np.ascontiguousarray(a, dtype=np.float64) for a in (num, dvds))
+    if num.shape != dvds.shape:
+        raise ValueError("num and dvds differ in shape")
+    out = np.empty((4,) + num.shape)
+    _check(load_library().pmx_check_force_mult(_dptr(num), _dptr(dvds), num.size, float(krad),
+                                               float(alpha), _dptr(out)), "check_force_mult")
+    return dict(zip(("power", "M", "power_general", "M_general"), out))
 
 
 def check_cooling(cfg: setups.WindConfig, rho, p, xi, dt, pre=None, device: bool = True) -> dict:
