@@ -1951,8 +1951,10 @@ int pmx_wind_create(const pmx_wind_desc* d, pmx_wind** out) {
         lf[LF_COS * sa + q] = cos(toff);
       }
   w->k.fast_div = fast_div ? 1 : 0;
+  // (lforce_bins forms a zone's byte offset in a table plane in 32 bits)
   w->k.lf_fast = fast_div && lf_geom && !w->k.fm_fast && w->k.fm_points == 0 &&
-                 fabs(k.alpharad) <= 2.0 && k.krad >= 0.0 && k.krad <= 0x1p100;
+                 w->sv < (1ll << 29) && fabs(k.alpharad) <= 2.0 && k.krad >= 0.0 &&
+                 k.krad <= 0x1p100;
 
   // pack the geometry tables into one buffer
   std::vector<std::pair<const double**, const std::vector<double>*>> parts = {
