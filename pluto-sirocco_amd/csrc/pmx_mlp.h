@@ -1,6 +1,6 @@
 // Device helpers of the MLP cooling surrogate: parameter layout, BF16
 // conversion, matrix-core fragments and the dense layers of a 16-sample
-// tile.  One 64-lane wavefront owns a tile.
+// tile (one 64-lane wavefront a tile; training has four).
 //
 // v_mfma_f32_16x16x16_bf16 operand layout (per lane l, r = l % 16,
 // q = l / 16): A[r][4q .. 4q+3], B[4q .. 4q+3][r], and the accumulator
@@ -52,10 +52,6 @@ __device__ __forceinline__ s4 frag(const unsigned short* p) {
 
 __device__ __forceinline__ float sigm(float z) { return 1.f / (1.f + expf(-z)); }
 __device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-  float s = sigm(z);
-  return s * (1.f + z * (1.f - s));
-}
 
 // raw features (log10 values) -> network inputs in [-1, 1] over the hull
 __device__ __forceinline__ void load_features(const float* x, float* xn) {
@@ -82,24 +78,15 @@ __device__ __forceinline__ void dense16(const unsigned short* in, const unsigned
   }
 }
 
-// bias + SiLU; stores the pre-activation (optional), the BF16 activation
-// [16][64] and its transpose [64][16] (optional)
-__device__ __forceinline__ void epilogue(const f4* acc, const float* b, float* Z, unsigned short* H,
-                                         unsigned short* HT, int l) {
+// bias + SiLU; stores the BF16 activation [16][64]
+__device__ __forceinline__ void epilogue(const f4* acc, const float* b, unsigned short* H, int l) {
   const int c = l & 15, r0 = (l >> 4) * 4;
 #pragma unroll
   for (int nt = 0; nt < 4; nt++) {
     const int n = nt * 16 + c;
     const float bn = b[n];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int s = r0 + i;
-      const float z = acc[nt][i] + bn;
-      if (Z) Z[s * 64 + n] = z;
-      const unsigned short hb = f2bf(silu(z));
-      H[s * 64 + n] = hb;
-      if (HT) HT[n * 16 + s] = hb;
-    }
+    for (int i = 0; i < 4; i++) H[(r0 + i) * 64 + n] = f2bf(silu(acc[nt][i] + bn));
   }
 }
 

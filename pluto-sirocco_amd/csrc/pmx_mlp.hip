@@ -403,13 +403,13 @@ __global__ __launch_bounds__(64) void mlp_predict_kernel(Weights w, const float*
   __syncthreads();
   f4 acc[4];
   dense16<16>(S.Xb, w.W1p, acc, l);
-  epilogue(acc, w.P + OFF_B1, nullptr, S.H1, nullptr, l);
+  epilogue(acc, w.P + OFF_B1, S.H1, l);
   __syncthreads();
   dense16<64>(S.H1, w.W2, acc, l);
-  epilogue(acc, w.P + OFF_B2, nullptr, S.H2, nullptr, l);
+  epilogue(acc, w.P + OFF_B2, S.H2, l);
   __syncthreads();
   dense16<64>(S.H2, w.W3, acc, l);
-  epilogue(acc, w.P + OFF_B3, nullptr, S.H3, nullptr, l);
+  epilogue(acc, w.P + OFF_B3, S.H3, l);
   __syncthreads();
   float y = output_unit(S.H3, w, l);
   if (l < 16 && valid) Yout[sidx] = y * YS;
@@ -584,13 +584,13 @@ __device__ __forceinline__ void surr_mlp_group(const Weights& wt, const SurrWork
   __syncthreads();
   f4 acc[4];
   dense16<16>(S.Xb, wt.W1p, acc, l);
-  epilogue(acc, wt.P + OFF_B1, nullptr, S.H1, nullptr, l);
+  epilogue(acc, wt.P + OFF_B1, S.H1, l);
   __syncthreads();
   dense16<64>(S.H1, wt.W2, acc, l);
-  epilogue(acc, wt.P + OFF_B2, nullptr, S.H2, nullptr, l);
+  epilogue(acc, wt.P + OFF_B2, S.H2, l);
   __syncthreads();
   dense16<64>(S.H2, wt.W3, acc, l);
-  epilogue(acc, wt.P + OFF_B3, nullptr, S.H3, nullptr, l);
+  epilogue(acc, wt.P + OFF_B3, S.H3, l);
   __syncthreads();
   float y = output_unit(S.H3, wt, l);
   if (l < 16) ylds[r] = y * YS;
