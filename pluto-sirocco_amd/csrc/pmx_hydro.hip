@@ -467,7 +467,7 @@ GhostLayout ghost_layout(const pmx_hydro* h) {
 // PLUTO's arrays are handed over in pieces through V[1], which holds nothing
 // between two steps, so a hand-over needs no memory of its own.  V[1] is made
 // long enough that a ghosted array of up to HANDOVER_MIN values goes in one
-// piece (64^3: 1.7 M values, a step with both transfers 2.05 ms); a piece is
+// piece (64^3: 1.7 M values, a step with both transfers 2.07 ms); a piece is
 // at most HANDOVER_MAX values, a launch of one thread each.
 constexpr long long HANDOVER_MIN = 1ll << 22, HANDOVER_MAX = 1ll << 28;
 
